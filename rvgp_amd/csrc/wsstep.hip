@@ -189,14 +189,23 @@ __device__ void wait_all(FlagOf flag_of, int n, int epoch, int* ctl) {
     __syncthreads();
 }
 
+// Every memory operation this wave has issued is complete.  An explicit
+// instruction: after a builtin wait the compiler knows of no store in flight
+// and drops the wait that belongs behind a release fence's L2 write-back,
+// so that the flag could overtake the write-back and a consumer read the
+// previous step's tile.
+__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // Every wave waits for its own stores to reach the L2 (vmcnt 0); after the
 // barrier one lane's agent-scope release fence writes the L2 back -- the
-// workgroup's waves share one CU and so one L2 -- and raises the flag.
+// workgroup's waves share one CU and so one L2 -- and, when that is done,
+// raises the flag.
 __device__ void publish(int* flag, int epoch) {
-    __builtin_amdgcn_s_waitcnt(0);
+    wait_vm();
     __syncthreads();
     if (threadIdx.x == 0) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        wait_vm();
         st_flag(flag, epoch);
     }
 }
