@@ -71,6 +71,30 @@ int rvgp_fps(const double* x, int n, int D, int n_iter, int start_idx, double sp
              int use_spacing, const double* diam2, double* ds, int* perm, double* lambdas,
              int* n_sel, void* stream);
 
+/* Spatial blocks of a point set: the points in the order of a space-filling curve, cut into blocks
+ * of 64 with their bounding boxes, so that whole blocks can be skipped.
+ *
+ * rvgp_morton_keys: keys (n) of the points' box coordinates Y (n, P <= 62, row
+ * stride ldy) quantised over [lo, hi] (P each, device); sorting them gives the
+ * curve order.  rvgp_blocks: the blocks of x (n, D <= 64) in `order` (a
+ * permutation, int64), P <= 6, into a buffer of rvgp_blocks_bytes(n, D, transposed)
+ * bytes; Y must be x itself (D <= 6) or an orthonormal projection of it (no
+ * distance in Y exceeds the one in x), lo / hi its column minima and maxima;
+ * transposed = 1 for rvgp_fps_blocks, 0 for rvgp_knn_blocks. */
+int rvgp_morton_keys(const double* Y, int ldy, int n, int P, const double* lo, const double* hi,
+                     long long* keys, void* stream);
+size_t rvgp_blocks_bytes(int n, int D, int transposed);
+int rvgp_blocks(const double* x, int n, int D, const double* Y, int ldy, int P, const double* lo,
+                const double* hi, const long long* order, int transposed, void* blocks,
+                size_t bytes, void* stream);
+
+/* rvgp_fps over spatial blocks (the same selections and distances, bit for
+ * bit): a selected point updates only the blocks whose box it can reach.
+ * n <= 262144, D <= 64; x, ds, perm, lambdas, n_sel as rvgp_fps. */
+int rvgp_fps_blocks(const double* x, const void* blocks, size_t bytes, int n, int D, int n_iter,
+                    int start_idx, double spacing, int use_spacing, const double* diam2, double* ds,
+                    int* perm, double* lambdas, int* n_sel, void* stream);
+
 /* ---------------------------------------------------------------------
  * a2  kNN graph  -- replaces geometry.manifold_graph(typ='knn')
  *     (RVGP/geometry.py:100-123: sklearn kneighbors_graph(include_self=False)

@@ -27,6 +27,10 @@ SIGNATURES = {
     "rvgp_last_error": (ctypes.c_char_p, []),
     "rvgp_fps_diam2": (I, [P, I, I, P, P]),
     "rvgp_fps": (I, [P, I, I, I, I, D, I, P, P, P, P, P, P]),
+    "rvgp_morton_keys": (I, [P, I, I, I, P, P, P, P]),
+    "rvgp_blocks_bytes": (S, [I, I, I]),
+    "rvgp_blocks": (I, [P, I, I, P, I, I, P, P, P, I, P, S, P]),
+    "rvgp_fps_blocks": (I, [P, P, S, I, I, I, I, D, I, P, P, P, P, P, P]),
     "rvgp_knn_ws_bytes": (S, [I, I]),
     "rvgp_knn": (I, [P, I, I, I, P, P, P, S, P]),
     "rvgp_affinity": (I, [P, I, I, D, P, I, P]),

@@ -16,25 +16,51 @@ depends on node order, run on the original numbering).
 """
 import torch
 
+from . import _lib
+
+BOX_DIMS = 6  # box coordinates per point (blocks.h)
+
+
+class SpatialOrder:
+    """The points X (n, D) along a Morton curve of their top min(D, dims)
+    principal coordinates (own_axes: of their own coordinates, D <= dims):
+    perm (new position -> old node), and the coordinates the curve was made
+    from, which bound distances from below."""
+
+    def __init__(self, X, dims=BOX_DIMS, own_axes=False):
+        P = min(X.shape[1], dims)
+        self.X, self.P = X, P
+        self.Y = X if own_axes else _principal(X, P)
+        self.lo, self.hi = torch.aminmax(self.Y, dim=0)
+        keys = torch.empty(X.shape[0], dtype=torch.int64, device=X.device)
+        _lib.call("rvgp_morton_keys", _lib.ptr(self.Y), self.Y.stride(0), X.shape[0], P,
+                  _lib.ptr(self.lo), _lib.ptr(self.hi), _lib.ptr(keys), _lib.stream())
+        self.perm = torch.sort(keys, stable=True).indices
+
+    def blocks(self, transposed):
+        """The points' spatial blocks (rvgp_blocks) as one byte tensor."""
+        n, D = self.X.shape
+        size = _lib.lib().rvgp_blocks_bytes(n, D, int(transposed))
+        out = torch.empty(size, dtype=torch.uint8, device=self.X.device)
+        _lib.call("rvgp_blocks", _lib.ptr(self.X), n, D, _lib.ptr(self.Y), self.Y.stride(0), self.P,
+                  _lib.ptr(self.lo), _lib.ptr(self.hi), _lib.ptr(self.perm), int(transposed),
+                  _lib.ptr(out), size, _lib.stream())
+        return out
+
+
+def _principal(X, P):
+    """The top-P principal coordinates of the points."""
+    from . import dense
+    Xc = (X - X.mean(0, keepdim=True)).contiguous()
+    C = dense.gemm_sym(Xc, Xc)
+    _, V = dense.syev(C)
+    return dense.gemm(Xc, V[:, -P:].contiguous())
+
 
 def morton_perm(X, max_dims=6):
     """Permutation (new position -> old node) sorting nodes by the Morton
     code of their top-P principal coordinates (P = min(D, max_dims))."""
-    from . import dense
-    Xc = (X - X.mean(0, keepdim=True)).contiguous()
-    C = dense.gemm_sym(Xc, Xc)
-    w, V = dense.syev(C)
-    P = min(X.shape[1], max_dims)
-    Y = dense.gemm(Xc, V[:, -P:].contiguous())
-    bits = min(20, 62 // P)
-    lo = Y.min(0).values
-    span = (Y.max(0).values - lo).clamp_min(1e-300)
-    q = ((Y - lo) / span * ((1 << bits) - 1)).round().to(torch.int64)
-    key = torch.zeros(X.shape[0], dtype=torch.int64, device=X.device)
-    for b in range(bits - 1, -1, -1):
-        for d in range(P):
-            key = (key << 1) | ((q[:, d] >> b) & 1)
-    return torch.sort(key, stable=True).indices
+    return SpatialOrder(X, max_dims).perm
 
 
 def bsr_permutation(rowptr, cols, perm):

@@ -1,0 +1,72 @@
+"""Spatial blocks: the farthest-point loop in registers and over blocks, against the oracle (bit for bit) at the sizes where their
+tiles, block counts and dispatch lines change."""
+import numpy as np
+import pytest
+
+from oracle import cpu
+from tests.util import flat_torus3, torus
+
+pytestmark = pytest.mark.gpu
+
+
+def _points(n, D, seed):
+    if D == 32:
+        return flat_torus3(n, seed)
+    x = torus(n, seed)
+    return np.concatenate([x, x * x], 1)[:, :D] if D > 3 else x[:, :D].copy()
+
+
+# registers: 256 R points, R = 2 ... 16; blocks: 128, 256, 512 testing threads
+@pytest.mark.parametrize("n,D,N", [(1, 3, 1), (63, 3, 63), (512, 3, 100), (513, 2, 100), (1025, 1, 70),
+                                   (1536, 3, 90), (2049, 3, 90), (2560, 3, 90), (3329, 3, 90),
+                                   (4096, 3, 150), (4097, 3, 150), (16384, 3, 100), (16385, 2, 64),
+                                   (512, 32, 120), (1300, 4, 200), (3000, 7, 80), (33000, 3, 70),
+                                   (66000, 3, 64)])
+def test_fps_forms_match_the_oracle(n, D, N):
+    from rvgp_amd import geometry
+    x = _points(n, D, n)
+    p, lam = geometry.furthest_point_sampling(x, N=N, start_idx=n // 2)
+    p_ref, lam_ref = cpu.fps(x, N=N, start_idx=n // 2)
+    np.testing.assert_array_equal(p, p_ref)
+    np.testing.assert_array_equal(lam, lam_ref)
+
+
+@pytest.mark.parametrize("n", [300, 4000, 5000])
+@pytest.mark.parametrize("scale", [1.0, 1e-160, 1e160])
+def test_fps_forms_break_ties_by_index(n, scale):
+    """Points of a small lattice, most of them several times over: equal and
+    nearly equal squares, distances of 0, squares that under- and overflow."""
+    from rvgp_amd import geometry
+    x = np.random.default_rng(n).integers(0, 8, (n, 3)) * (0.1 * scale)
+    p, lam = geometry.furthest_point_sampling(x, N=n // 4)
+    p_ref, lam_ref = cpu.fps(x, N=n // 4)
+    np.testing.assert_array_equal(p, p_ref)
+    np.testing.assert_array_equal(lam, lam_ref)
+
+
+@pytest.mark.parametrize("n", [3000, 6000])
+def test_fps_forms_stop_at_the_spacing(n):
+    from rvgp_amd import geometry
+    x = torus(n, 5)
+    p, lam = geometry.furthest_point_sampling(x, spacing=0.04)
+    p_ref, lam_ref = cpu.fps(x, spacing=0.04)
+    np.testing.assert_array_equal(p, p_ref)
+    np.testing.assert_array_equal(lam, lam_ref)
+
+
+@pytest.mark.parametrize("P", [1, 3, 6, 7])
+def test_morton_keys_are_the_interleaved_quantised_coordinates(P):
+    import torch
+    from rvgp_amd import _lib
+    Y = torch.as_tensor(np.random.default_rng(P).normal(size=(1000, P)), device="cuda")
+    lo, hi = torch.aminmax(Y, dim=0)
+    keys = torch.empty(1000, dtype=torch.int64, device="cuda")
+    _lib.call("rvgp_morton_keys", _lib.ptr(Y), P, 1000, P, _lib.ptr(lo), _lib.ptr(hi), _lib.ptr(keys),
+              _lib.stream())
+    bits = min(20, 62 // P)
+    q = ((Y - lo) / (hi - lo) * ((1 << bits) - 1)).round().to(torch.int64)
+    ref = torch.zeros(1000, dtype=torch.int64, device="cuda")
+    for b in range(bits - 1, -1, -1):
+        for d in range(P):
+            ref = (ref << 1) | ((q[:, d] >> b) & 1)
+    assert torch.equal(keys, ref)
