@@ -71,7 +71,8 @@ int rvgp_fps(const double* x, int n, int D, int n_iter, int start_idx, double sp
              int use_spacing, const double* diam2, double* ds, int* perm, double* lambdas,
              int* n_sel, void* stream);
 
-/* Spatial blocks of a point set: the points in the order of a space-filling curve, cut into blocks
+/* Spatial blocks of a point set, shared by the farthest-point loop and the
+ * kNN scan: the points in the order of a space-filling curve, cut into blocks
  * of 64 with their bounding boxes, so that whole blocks can be skipped.
  *
  * rvgp_morton_keys: keys (n) of the points' box coordinates Y (n, P <= 62, row
@@ -114,6 +115,11 @@ int rvgp_fps_blocks(const double* x, const void* blocks, size_t bytes, int n, in
 size_t rvgp_knn_ws_bytes(int n, int k);
 int rvgp_knn(const double* x, int n, int D, int k, const int* qperm, int* nbr, void* ws,
              size_t ws_bytes, void* stream);
+
+/* rvgp_knn over spatial blocks: the same nbr (n, k), from the candidate
+ * blocks whose box can hold a neighbour.  0 < k < n, k <= 64, D <= 64; finite
+ * points. */
+int rvgp_knn_blocks(const void* blocks, size_t bytes, int n, int D, int k, int* nbr, void* stream);
 
 /* Dense Gaussian affinity of manifold_graph(typ='affinity')
  * (geometry.py:114-118): A (n x n, row stride lda) with

@@ -31,6 +31,7 @@ SIGNATURES = {
     "rvgp_blocks_bytes": (S, [I, I, I]),
     "rvgp_blocks": (I, [P, I, I, P, I, I, P, P, P, I, P, S, P]),
     "rvgp_fps_blocks": (I, [P, P, S, I, I, I, I, D, I, P, P, P, P, P, P]),
+    "rvgp_knn_blocks": (I, [P, S, I, I, I, P, P]),
     "rvgp_knn_ws_bytes": (S, [I, I]),
     "rvgp_knn": (I, [P, I, I, I, P, P, P, S, P]),
     "rvgp_affinity": (I, [P, I, I, D, P, I, P]),

@@ -18,7 +18,7 @@ import torch
 from . import _lib, geometry
 from .eigsolve import chfsi
 from .ptu_dijkstra import connections_device, tangent_frames_device
-from .reorder import bsr_permutation, morton_perm, permute_bsr
+from .reorder import SpatialOrder, bsr_permutation, permute_bsr
 from .smoothing import lambda_min_lower, vector_diffusion_device, vector_diffusion_spectral_device
 from .sparse import BSR, graph_laplacian
 
@@ -49,8 +49,8 @@ class data:
         # Morton renumbering of the leading principal coordinates: groups
         # manifold neighbours into the kNN's waves and, below, gives the
         # block SpMM its locality
-        perm = morton_perm(Xd)
-        G = geometry.manifold_graph(Xd, n_neighbors=n_neighbors, query_order=perm)
+        order = SpatialOrder(Xd)
+        G = geometry.manifold_graph(Xd, n_neighbors=n_neighbors, query_order=order)
         if isinstance(vertices, np.ndarray):
             G._positions = vertices
         sync()
@@ -63,7 +63,7 @@ class data:
         # on latency-bound steps (heap walks, small eigenproblems, host round
         # trips).
         kL = N if n_eigenpairs is None else min(int(n_eigenpairs), N)
-        perm = perm if reorder else None
+        perm = order.perm if reorder else None
         t0 = time.perf_counter()
         Lb = graph_laplacian(G)
         # the renumbered pattern, shared by both Laplacians of the graph

