@@ -53,6 +53,9 @@ constexpr int TT = TB * TB;     // doubles per tile
 constexpr int NTH = 256;        // threads per task workgroup (4 waves)
 constexpr int LDT = TB + 1;     // LDS tile row stride
 constexpr int kSpinLimit = 1 << 21;
+// Filter values that an optimiser's trial step sends to 0 (a sigma_f of 1e-300,
+// a steep filter): 1 / S stays finite, S itself is as good as 0.
+constexpr double kMinS = 1e-280;
 
 // task numbering.  L column j: the diagonal task (which also produces
 // L(j+1,j)), then L(i,j) for i >= j+2; X column j: X(i,j) for i > j.
@@ -111,6 +114,7 @@ struct StepArgs {
     const double* G;
     const double* b;
     const double* yy;
+    const double* c;  // y = Phi c + e with Phi^T e = 0, yy = |e|^2; or NULL
     const double* lower;
     double* u;
     const int* trainable;
@@ -419,7 +423,7 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
         if (row < a.k) {
             double r, dn, dk;
             filter_terms(a.typ, a.lam[row], nu, kappa, r, dn, dk);
-            add = s2 / (sf * a.n_rows * r / sr);
+            add = s2 / fmax(sf * a.n_rows * r / sr, kMinS);
         }
         dadd[tid] = add;
     }
@@ -582,7 +586,7 @@ __device__ void task_filter(const StepArgs& a, const Layout& g, int epoch, doubl
     for (int q = tid; q < k; q += NTH) {
         double r, dn, dk;
         filter_terms(a.typ, a.lam[q], nu, kappa, r, dn, dk);
-        const double v = sf * a.n_rows * r / sr;
+        const double v = fmax(sf * a.n_rows * r / sr, kMinS);
         S[q] = v;
         dS[q] = v * (dn - snu);
         dS[k + q] = v * (dk - ska);
@@ -629,6 +633,11 @@ __device__ void task_row(const StepArgs& a, const Layout& g, int i, int epoch) {
 //   P[0] = sum b_q w_q       P[1] = sum w_q^2 / S_q    P[2] = sum A^-1_qq / S_q
 //   P[3] = sum log L_qq      P[4..6] = sum gS_q dS_q/d(nu, kappa, sigma_f)
 // with gS_q = (1/S_q - s2 A^-1_qq / S_q^2 - w_q^2 / S_q^2) / 2.
+// With the split y = Phi c + e, Phi^T e = 0 (a.c), p_q = w_q / S_q is
+// (Phi^T K_y^-1 y)_q and the first two become
+//   P[0] = sum c_q p_q          (y^T K_y^-1 y = P[0] + |e|^2 / s2)
+//   P[1] = sum p_q (c_q - w_q) / s2   (|K_y^-1 y|^2 = P[1] + |e|^2 / s2^2),
+// where y^T y - b^T w of the other form cancels to s2 times its terms.
 __device__ void task_col(const StepArgs& a, const Layout& g, int j, int epoch, double* lds) {
     const int tid = threadIdx.x, T = g.T, k = a.k;
     int* sync = a.sync;
@@ -668,9 +677,10 @@ __device__ void task_col(const StepArgs& a, const Layout& g, int j, int epoch, d
             const double s2 = softplus_d(a.u[3]) + a.lower[3];
             const double S = a.ws[g.oS + qq];
             const double* dS = a.ws + g.oDS;
-            const double gS = 0.5 * (1.0 / S - s2 * av / (S * S) - w * w / (S * S));
-            v[0] = a.b[qq] * w;
-            v[1] = w * w / S;
+            const double p = w / S;
+            const double gS = 0.5 * ((1.0 - s2 * av / S) / S - p * p);
+            v[0] = a.c != nullptr ? a.c[qq] * p : a.b[qq] * w;
+            v[1] = a.c != nullptr ? p * ((a.c[qq] - w) / s2) : w * p;
             v[2] = av / S;
             v[3] = log(a.ws[g.oL + (size_t)tix(j, j) * TT + tid * TB + tid]);
             v[4] = gS * dS[qq];
@@ -709,11 +719,13 @@ __device__ void task_final(const StepArgs& a, const Layout& g, int epoch) {
         const double s2 = softplus_d(a.u[3]) + a.lower[3];
         const double y2 = a.yy[0], M = a.M;
         const double two_pi = 6.283185307179586;
-        const double nlml = 0.5 * (y2 - bw) / s2 + 0.5 * ((M - k) * log(s2) + lS + 2.0 * ld) +
-                            0.5 * M * log(two_pi);
+        // y^T K_y^-1 y and |K_y^-1 y|^2
+        const double ya = a.c != nullptr ? bw + y2 / s2 : (y2 - bw) / s2;
         const double wGw = bw - s2 * ww;
-        const double res2 = y2 - 2.0 * bw + wGw;
-        const double gs2 = 0.5 * ((M - k) / s2 + tr - res2 / (s2 * s2));
+        const double aa = a.c != nullptr ? ww + y2 / (s2 * s2) : (y2 - 2.0 * bw + wGw) / (s2 * s2);
+        const double nlml = 0.5 * ya + 0.5 * ((M - k) * log(s2) + lS + 2.0 * ld) +
+                            0.5 * M * log(two_pi);
+        const double gs2 = 0.5 * ((M - k) / s2 + tr - aa);
         const double gr[4] = {P[4], P[5], P[6], gs2};
         const double up = a.u[p];
         const double sig = 1.0 / (1.0 + exp(-up));
@@ -797,12 +809,11 @@ extern "C" size_t rvgp_ws_step_sync_ints(int k) {
     return (size_t)make_layout(k).nsync;
 }
 
-extern "C" int rvgp_ws_step(int k, int typ, const double* evals, double n_rows, const double* G,
-                            int ldg, const double* b, const double* yy, double M,
-                            const double* lower, double* u, const int* trainable, double* m1,
-                            double* m2, double* t, int do_adam, double lr, double b1, double b2,
-                            double eps, void* ws, size_t ws_bytes, int* sync, size_t sync_ints,
-                            double* out, int* status, void* stream) {
+static int ws_step(const double* c, int k, int typ, const double* evals, double n_rows, const double* G,
+                   int ldg, const double* b, const double* yy, double M, const double* lower,
+                   double* u, const int* trainable, double* m1, double* m2, double* t, int do_adam,
+                   double lr, double b1, double b2, double eps, void* ws, size_t ws_bytes, int* sync,
+                   size_t sync_ints, double* out, int* status, void* stream) {
     RVGP_CHECK_ARG(k >= 1 && k <= RVGP_WS_STEP_MAX_K, "rvgp_ws_step: need 1 <= k <= %d",
                    RVGP_WS_STEP_MAX_K);
     RVGP_CHECK_ARG(ldg >= k, "rvgp_ws_step: ldg < k");
@@ -817,6 +828,7 @@ extern "C" int rvgp_ws_step(int k, int typ, const double* evals, double n_rows, 
     a.typ = typ;
     a.ldg = ldg;
     a.do_adam = do_adam;
+    a.c = c;
     a.n_rows = n_rows;
     a.M = M;
     a.lr = lr;
@@ -840,4 +852,25 @@ extern "C" int rvgp_ws_step(int k, int typ, const double* evals, double n_rows, 
     hipLaunchKernelGGL(ws_step_kernel, dim3(g.nblocks), dim3(NTH), 0, as_stream(stream), a);
     RVGP_LAUNCH_CHECK();
     return RVGP_OK;
+}
+
+extern "C" int rvgp_ws_step(int k, int typ, const double* evals, double n_rows, const double* G,
+                            int ldg, const double* b, const double* yy, double M,
+                            const double* lower, double* u, const int* trainable, double* m1,
+                            double* m2, double* t, int do_adam, double lr, double b1, double b2,
+                            double eps, void* ws, size_t ws_bytes, int* sync, size_t sync_ints,
+                            double* out, int* status, void* stream) {
+    return ws_step(nullptr, k, typ, evals, n_rows, G, ldg, b, yy, M, lower, u, trainable, m1, m2, t, do_adam,
+                   lr, b1, b2, eps, ws, ws_bytes, sync, sync_ints, out, status, stream);
+}
+
+extern "C" int rvgp_coef_step(int k, int typ, const double* evals, double n_rows, const double* G,
+                              int ldg, const double* b, const double* c, const double* ee,
+                              double M, const double* lower, double* u, const int* trainable, double* m1,
+                              double* m2, double* t, int do_adam, double lr, double b1, double b2,
+                              double eps, void* ws, size_t ws_bytes, int* sync, size_t sync_ints,
+                              double* out, int* status, void* stream) {
+    RVGP_CHECK_ARG(c != nullptr, "rvgp_coef_step: c is NULL");
+    return ws_step(c, k, typ, evals, n_rows, G, ldg, b, ee, M, lower, u, trainable, m1, m2, t, do_adam,
+                   lr, b1, b2, eps, ws, ws_bytes, sync, sync_ints, out, status, stream);
 }

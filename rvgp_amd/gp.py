@@ -7,9 +7,13 @@ hand-written adjoint here) and predict_f.
 Two exact forms of the same model y ~ N(0, Phi diag(S) Phi^T + s2 I):
   * function space: M x M Gram on the matrix cores (rvgp_gemm with the
     spectral filter as k-scale), blocked Cholesky, triangular solves;
-    in mixed precision alpha comes from the FP64 k x k system below
-    (Woodbury), refined against the matrix-free FP64 K_y, and no M x M
-    matrix is formed.
+    with at least twice as many rows as features (or in mixed precision) no
+    M x M matrix is formed: with y = Phi c + e, Phi^T e = 0, split once per
+    training set, and w of the FP64 k x k system below, p = Phi^T K_y^-1 y =
+    w / S, y^T K_y^-1 y = c^T p + |e|^2 / s2 and |K_y^-1 y|^2 = p^T (c - w) / s2
+    + |e|^2 / s2^2, without the weight form's y^T y - b^T w, which cancels at
+    small noise; a mixed fit with fewer rows solves by Woodbury, refined
+    against the matrix-free FP64 K_y.
   * weight space (Woodbury / determinant lemma): k x k system
     A = s2 S^-1 + Phi^T Phi; G = Phi^T Phi and b = Phi^T y are formed once per
     training set, so an optimiser step costs O(k^3) and never touches an
@@ -80,6 +84,17 @@ def weight_space_stats(U, c, precision="fp64"):
 
 
 FUSED_STEP_MAX_K = 2048  # RVGP_WS_STEP_MAX_K
+# A function-space fit of M rows works on the k x k system from M = 2 k on.
+# Its flops are ~(k / M)^3 of the M x M factorisation's; below 2 k rows
+# Phi^T Phi is singular for the tangent fields' frames (rank m d < M).
+# M = 4731, k = 200: an evaluation 10.0 -> 0.14 ms, building
+# the engine 0.84 ms.  Its
+# error against 80-bit arithmetic, noise 1 ... 1e-6, data with noise: NLML <=
+# 4e-13 and gradient <= 5e-13 (M x M: 1e-8 and 3e-8), mean 2e-13 (7e-8),
+# variance 1e-13 (5e-7); without noise, s2 -> 1e-6: gradient 1e-9 (2e-12), the
+# others as before or better.
+COEF_MIN_ROWS = 2
+SPLIT_RIDGE = 1e-12  # of the largest diagonal entry of Phi^T Phi
 
 
 class GPREngine:
@@ -113,28 +128,24 @@ class GPREngine:
         self.lower = torch.as_tensor(np.asarray(lower, np.float64), device=dev)
         self.theta = torch.zeros(3, **f64)
         self.s2 = torch.zeros(1, **f64)
-        self.S = torch.empty(self.k, **f64)
-        self.dS = torch.empty(3 * self.k, **f64)
-        self.gS = torch.empty(self.k, **f64)
-        self.out = torch.zeros(9, **f64)
-        self.status = torch.zeros(1, dtype=torch.int32, device=dev)
-        self.fused_step = True
+        self._scalars()
         self.ya = torch.zeros(1, **f64)
         self.aa = torch.zeros(1, **f64)
         self._dot_ws = torch.empty(
             _lib.lib().rvgp_dot_ws_bytes(self.M * self.R) // 8 + 1, **f64)
         self._cs_ws = torch.empty(
             _lib.lib().rvgp_colsumsq_ws_bytes(max(self.M, self.k), max(self.k, 1)) // 8 + 1, **f64)
-        if self.form == "weight" or precision == "mixed":
-            # k x k normal-equation system (weight space; in the mixed
-            # function-space form it carries log det, diag(Phi^T K^-1 Phi) and
-            # the Woodbury solve for alpha, all in FP64)
+        # k x k normal-equation system: weight space; in the function-space
+        # forms it carries log det, diag(Phi^T K^-1 Phi) and the solve for
+        # alpha, all in FP64
+        tall = self.form == "function" and self.M >= COEF_MIN_ROWS * self.k
+        self.normal = self.form == "weight" or precision == "mixed" or tall
+        if self.normal:
             if gram_mode is None:
                 # mixed weight form: FP32 Phi tiles, products accumulated in
                 # FP64 on the matrix cores (an FP32-accumulated G over M = 768k
-                # rows costs ~1e-4 in the NLML).  The function form's Woodbury
-                # refinement divides by s2, which amplifies the ~1e-7 error of
-                # FP32-rounded rows until it stops converging at s2 ~ 1e-5; its
+                # rows costs ~1e-4 in the NLML).  The function forms divide by
+                # s2, which amplifies the ~1e-7 error of FP32-rounded rows; their
                 # G (M <= fs_max rows) costs next to nothing in FP64.
                 mixed_rows = precision == "mixed" and self.form == "weight"
                 gram_mode = dense.GEMM_F32_ACC64 if mixed_rows else dense.GEMM_F64
@@ -146,20 +157,72 @@ class GPREngine:
             self.G = G.double().contiguous()
             self.G = 0.5 * (self.G + self.G.T)
             self.b = dense.gemm(self.Phi, self.y, transA=True)
+            self.coef = tall and gram_mode == dense.GEMM_F64 and self._split_rows()
+            self.normal = self.coef or self.form == "weight" or precision == "mixed"
+        if self.normal:
             self.yy = torch.empty(1, **f64)
             self._dot(self.y, self.y, self.yy)
-            self.A = torch.empty((self.k, self.k), **f64)
-            self.w = torch.empty((self.k, self.R), **f64)
-            self.Linv = torch.empty((self.k, self.k), **f64)
-            self.eye = torch.eye(self.k, **f64)
-            self.ainv = torch.empty(self.k, **f64)
+            self._system()
         if self.form == "function":
-            if precision != "mixed":
+            if not self.normal:
                 self.K = torch.empty((self.M, self.M), **f64)
-            self.a = torch.empty((self.M, self.R), **f64)
-            self.Z = torch.empty_like(self.Phi)
+            if not self.coef:
+                self.a = torch.empty((self.M, self.R), **f64)
+                self.Z = torch.empty_like(self.Phi)
             self.q = torch.empty(self.k, **f64)
             self.logdet = torch.empty(1, **f64)
+
+    def _scalars(self):
+        """Buffers every form uses.  The outputs and the status word share one
+        allocation, so that a host optimiser reads both in one copy."""
+        f64 = dict(dtype=torch.float64, device=self.dev)
+        self.S = torch.empty(self.k, **f64)
+        self.dS = torch.empty(3 * self.k, **f64)
+        self.gS = torch.empty(self.k, **f64)
+        self._result = torch.zeros(10, **f64)
+        self.out = self._result[:9]
+        self.status = self._result[9:].view(torch.int32)[:1]
+        self.fused_step = True
+        self.coef = False
+
+    def _system(self):
+        """Buffers of the k x k system, and of the single-launch step where it
+        serves this fit."""
+        f64 = dict(dtype=torch.float64, device=self.dev)
+        self.A = torch.empty((self.k, self.k), **f64)
+        self.w = torch.empty((self.k, self.R), **f64)
+        self.Linv = torch.empty((self.k, self.k), **f64)
+        self.eye = torch.eye(self.k, **f64)
+        self.ainv = torch.empty(self.k, **f64)
+        if self.fused():
+            L = _lib.lib()
+            self._fws = torch.empty(L.rvgp_ws_step_ws_bytes(self.k) // 8, **f64)
+            # flags of the dataflow: zeroed once, then advanced by every call
+            self._fsync = torch.zeros(L.rvgp_ws_step_sync_ints(self.k), dtype=torch.int32,
+                                      device=self.dev)
+
+    def _split_rows(self):
+        """y = Phi c + e with Phi^T e = 0: c (k, R) and |e|^2, by the Cholesky
+        factor of G with a ridge, three passes against the rows.  Duplicated
+        features and fewer tangent rows than features leave G singular: the
+        ridge makes it solvable, the passes take the ridge's share out of every
+        direction the rows hold, and any c with the right Phi c serves.  False
+        when G is not positive definite even so."""
+        L = self.G + (SPLIT_RIDGE * torch.diagonal(self.G).max()) * torch.eye(
+            self.k, dtype=torch.float64, device=self.dev)
+        _, st = dense.potrf(L, check=False)
+        if int(st.item()) != 0:
+            return False
+        c, e = torch.zeros_like(self.b), self.y
+        for _ in range(3):
+            r = dense.gemm(self.Phi, e, transA=True)
+            dense.trsm(L, r)
+            dense.trsm(L, r, trans=True)
+            c = c + r
+            e = (self.y - dense.gemm(self.Phi, c)).contiguous()
+        self.c, self.ee = c.contiguous(), torch.empty(1, dtype=torch.float64, device=self.dev)
+        self._dot(e, e, self.ee)
+        return True
 
     def _init_from_stats(self, stats, evals, n_rows, typ, form, precision, lower):
         G, b, yy, M = stats
@@ -186,19 +249,11 @@ class GPREngine:
         self.lower = torch.as_tensor(np.asarray(lower, np.float64), device=dev)
         self.theta = torch.zeros(3, **f64)
         self.s2 = torch.zeros(1, **f64)
-        self.S = torch.empty(self.k, **f64)
-        self.dS = torch.empty(3 * self.k, **f64)
-        self.gS = torch.empty(self.k, **f64)
-        self.out = torch.zeros(9, **f64)
-        self.status = torch.zeros(1, dtype=torch.int32, device=dev)
-        self.fused_step = True
+        self.normal = True
+        self._scalars()
         self._cs_ws = torch.empty(
             _lib.lib().rvgp_colsumsq_ws_bytes(self.k, self.k) // 8 + 1, **f64)
-        self.A = torch.empty((self.k, self.k), **f64)
-        self.w = torch.empty((self.k, self.R), **f64)
-        self.Linv = torch.empty((self.k, self.k), **f64)
-        self.eye = torch.eye(self.k, **f64)
-        self.ainv = torch.empty(self.k, **f64)
+        self._system()
 
     # ---------------------------------------------------------------- params
     def set_theta(self, theta):
@@ -230,11 +285,19 @@ class GPREngine:
     # ---------------------------------------------------------------- evaluate
     def evaluate(self):
         """Enqueue NLML + gradient; results in self.out (device):
-        [nlml, d/d(nu, kappa, sigma_f, s2), d/du(...)]."""
+        [nlml, d/d(nu, kappa, sigma_f, s2), d/du(...)].  One launch where the
+        single-launch step serves the fit (k = 500: 216 against 358 us)."""
+        return self._ws_step(0) if self.fused() else self._evaluate_state()
+
+    def _evaluate_state(self):
+        """evaluate() by the multi-kernel path, which leaves the factors and
+        solutions that predictions read (A, w; K, a) behind."""
         self._prologue()
         s = _lib.stream()
         self.status.zero_()
-        if self.form == "weight" or self.precision == "mixed":
+        if self.normal:
+            if self.coef:
+                self.S.clamp_(min=1e-280)  # a filter value of 0: 1 / S stays finite
             _lib.call("rvgp_ws_form", self.k, _lib.ptr(self.G), self.k, _lib.ptr(self.S),
                       _lib.ptr(self.s2), _lib.ptr(self.A), self.k, s)
             _lib.call("rvgp_potrf", 1, self.k, _lib.ptr(self.A), self.k, _lib.ptr(self.status), s)
@@ -251,35 +314,42 @@ class GPREngine:
                       _lib.ptr(self.ainv), _lib.ptr(self.b), _lib.ptr(self.w), _lib.ptr(Gw),
                       _lib.ptr(self.yy), _lib.ptr(self.S), _lib.ptr(self.dS), _lib.ptr(self.s2),
                       _lib.ptr(self.u), _lib.ptr(self.gS), _lib.ptr(self.out), s)
-        else:
-            if self.precision == "mixed":
-                # alpha = K_y^-1 y = (y - Phi w) / s2 (Woodbury; w = A^-1 Phi^T y
-                # above), then two refinement sweeps against the FP64 K_y
-                torch.div(self.y - dense.gemm(self.Phi, self.w), self.s2, out=self.a)
-                for _ in range(2):
-                    self.a += self._woodbury(self.y - self._apply_Ky(self.a))
-                self._dot(self.y, self.a, self.ya)
-            else:
-                self._factor()
-                # a = K_y^-1 y: L^-1 y first (ya = |L^-1 y|^2), then L^-T
-                self.a.copy_(self.y)
-                dense.trsm(self.K, self.a)
-                self._dot(self.a, self.a, self.ya)
-                dense.trsm(self.K, self.a, trans=True)
+            return self.out
+        if self.coef:
+            p = (self.w / self.S.reshape(-1, 1)).contiguous()  # Phi^T K_y^-1 y
+            self._dot(self.c, p, self.ya)
+            self._dot(p, ((self.c - self.w) / self.s2).contiguous(), self.aa)
+            self.ya += self.ee / self.s2
+            self.aa += self.ee / (self.s2 * self.s2)
+        elif self.precision == "mixed":
+            # alpha = K_y^-1 y = (y - Phi w) / s2 (Woodbury; w = A^-1 Phi^T y
+            # above), then two refinement sweeps against the FP64 K_y
+            torch.div(self.y - dense.gemm(self.Phi, self.w), self.s2, out=self.a)
+            for _ in range(2):
+                self.a += self._woodbury(self.y - self._apply_Ky(self.a))
+            self._dot(self.y, self.a, self.ya)
             self._dot(self.a, self.a, self.aa)
-            if self.precision == "mixed":
-                _lib.call("rvgp_lemma_terms", self.k, float(self.M), _lib.ptr(self.S),
-                          _lib.ptr(self.s2), _lib.ptr(self.ainv), _lib.ptr(self.A), self.k,
-                          _lib.ptr(self.q), _lib.ptr(self.logdet), s)
-            else:
-                self.Z.copy_(self.Phi)
-                dense.trsm(self.K, self.Z)
-                self._colsumsq(self.Z, self.q)
             p = dense.gemm(self.Phi, self.a, transA=True)  # (k, R)
-            _lib.call("rvgp_fs_finish", self.k, float(self.M), self.R, _lib.ptr(self.q), _lib.ptr(p),
-                      _lib.ptr(self.ya), _lib.ptr(self.aa), _lib.ptr(self.logdet), _lib.ptr(self.S),
-                      _lib.ptr(self.dS), _lib.ptr(self.s2), _lib.ptr(self.u), _lib.ptr(self.gS),
-                      _lib.ptr(self.out), s)
+        else:
+            self._factor()
+            # a = K_y^-1 y: L^-1 y first (ya = |L^-1 y|^2), then L^-T
+            self.a.copy_(self.y)
+            dense.trsm(self.K, self.a)
+            self._dot(self.a, self.a, self.ya)
+            dense.trsm(self.K, self.a, trans=True)
+            self._dot(self.a, self.a, self.aa)
+            self.Z.copy_(self.Phi)
+            dense.trsm(self.K, self.Z)
+            self._colsumsq(self.Z, self.q)
+            p = dense.gemm(self.Phi, self.a, transA=True)  # (k, R)
+        if self.normal:
+            _lib.call("rvgp_lemma_terms", self.k, float(self.M), _lib.ptr(self.S),
+                      _lib.ptr(self.s2), _lib.ptr(self.ainv), _lib.ptr(self.A), self.k,
+                      _lib.ptr(self.q), _lib.ptr(self.logdet), s)
+        _lib.call("rvgp_fs_finish", self.k, float(self.M), self.R, _lib.ptr(self.q), _lib.ptr(p),
+                  _lib.ptr(self.ya), _lib.ptr(self.aa), _lib.ptr(self.logdet), _lib.ptr(self.S),
+                  _lib.ptr(self.dS), _lib.ptr(self.s2), _lib.ptr(self.u), _lib.ptr(self.gS),
+                  _lib.ptr(self.out), s)
         return self.out
 
     # function-space helpers -------------------------------------------------
@@ -313,9 +383,11 @@ class GPREngine:
 
     # ---------------------------------------------------------------- host API
     def nlml_grad_u(self, u):
-        self.u.copy_(torch.as_tensor(np.asarray(u, np.float64), device=self.dev))
-        out = self.evaluate().cpu().numpy()
-        if int(self.status.item()) != 0:
+        self.u.copy_(torch.from_numpy(np.array(u, np.float64)))
+        self.evaluate()
+        res = self._result.cpu()
+        out = res[:9].numpy()
+        if int(res[9:].view(torch.int32)[0]) != 0:
             raise dense.CholeskyError("Cholesky decomposition was not successful: the GP system "
                                       "matrix is not positive definite")
         return float(out[0]), out[5:9].copy(), out
@@ -324,10 +396,10 @@ class GPREngine:
         """Mean (m*,) -- (m*, R) with R right-hand sides -- and marginal
         variance (m*,) of f at rows Phi_star, as GPflow's
         GPR.predict_f(full_cov=False) (the variance does not depend on y)."""
-        self.evaluate()
+        self._evaluate_state()
         Ps = Phi_star.to(torch.float64).contiguous()
         m = Ps.shape[0]
-        if self.form == "weight" or self.precision == "mixed":
+        if self.normal:
             # mean = Phi* w, var = s2 |L_A^-1 phi*|^2 from the FP64 k x k system
             mean = dense.gemm(Ps, self.w)
             Zt = Ps.T.contiguous()
@@ -361,9 +433,9 @@ class GPREngine:
         mean_i = T_i (U_i w) and var_ip = s2 T_i[p] B_i T_i[p]^T with
         B_i = (L_A^-1 U_i^T)^T (L_A^-1 U_i^T) (d x d), so the triangular solve
         runs on m*d columns instead of m*D.  Weight-space system only."""
-        if not (self.form == "weight" or self.precision == "mixed"):
+        if not self.normal:
             raise ValueError("predict_nodes needs the k x k weight-space system")
-        self.evaluate()
+        self._evaluate_state()
         m, D, d = T_star.shape
         T = T_star.to(torch.float64).contiguous()
         mu = dense.gemm(U_star, self.w)                                  # (m*d, R)
@@ -401,23 +473,19 @@ class GPREngine:
 
     def fused(self):
         """Whether a step runs as the single-launch tile dataflow
-        (rvgp_ws_step): weight form, one right-hand side, k <= 2048."""
-        return (self.fused_step and self.form == "weight" and self.R == 1
+        (rvgp_ws_step, rvgp_coef_step): weight form, or function form on the
+        k x k system; one right-hand side, k <= 2048."""
+        return (self.fused_step and (self.form == "weight" or self.coef) and self.R == 1
                 and self.k <= FUSED_STEP_MAX_K)
 
     def _ws_step(self, do_adam, lr=0.0, b1=0.9, b2=0.999, eps=1e-8):
-        if getattr(self, "_fws", None) is None:
-            L = _lib.lib()
-            self._fws = torch.empty(L.rvgp_ws_step_ws_bytes(self.k) // 8, dtype=torch.float64,
-                                    device=self.dev)
-            # flags of the dataflow: zeroed once, then advanced by every call
-            self._fsync = torch.zeros(L.rvgp_ws_step_sync_ints(self.k), dtype=torch.int32,
-                                      device=self.dev)
         args = (_lib.ptr(self.m1), _lib.ptr(self.m2), _lib.ptr(self.t),
                 _lib.ptr(self.trainable)) if do_adam else (None, None, None, None)
         m1, m2, t, tr = args
-        _lib.call("rvgp_ws_step", self.k, self.typ, _lib.ptr(self.evals), self.n_rows,
-                  _lib.ptr(self.G), self.G.stride(0), _lib.ptr(self.b), _lib.ptr(self.yy),
+        y = (self.b, self.c, self.ee) if self.coef else (self.b, self.yy)
+        _lib.call("rvgp_coef_step" if self.coef else "rvgp_ws_step", self.k, self.typ,
+                  _lib.ptr(self.evals), self.n_rows, _lib.ptr(self.G), self.G.stride(0),
+                  *[_lib.ptr(t) for t in y],
                   float(self.M), _lib.ptr(self.lower), _lib.ptr(self.u), tr, m1, m2, t,
                   int(do_adam), float(lr), float(b1), float(b2), float(eps), _lib.ptr(self._fws),
                   self._fws.numel() * 8, _lib.ptr(self._fsync), self._fsync.numel(),
@@ -430,13 +498,12 @@ class GPREngine:
         self.m2 = torch.zeros(4, **f64)
         self.t = torch.zeros(1, **f64)
         self.trainable = torch.as_tensor(np.asarray(trainable, np.int32), device=self.dev)
-        if self.fused():
-            self._ws_step(0)  # allocates the dataflow's workspace before any capture
 
     def adam_step(self, lr=0.05, b1=0.9, b2=0.999, eps=1e-8):
         """One device-resident optimiser step: NLML, adjoint, Adam update.
         No host synchronisation, so it can be captured in a HIP graph.  In the
-        weight form with one right-hand side the whole step is one launch."""
+        weight and coefficient forms with one right-hand side the whole step is one
+        launch."""
         if self.fused():
             self._ws_step(1, lr, b1, b2, eps)
             return

@@ -91,7 +91,7 @@ class manifold_GPR:
             nodes = nodes.cpu().numpy()
         nodes = torch.as_tensor(checked_nodes(nodes, data.n), device=self.engine.dev)
         e = self.engine
-        weight = hasattr(e, "predict_nodes") and (e.form == "weight" or e.precision == "mixed")
+        weight = hasattr(e, "predict_nodes") and e.normal
         U = data.intrinsic_rows(nodes) if weight else None
         if U is None:
             return self.predict_f(data.phi_rows(nodes.int()))
