@@ -284,9 +284,24 @@ __global__ __launch_bounds__(FT) void ws_finish_kernel(int k, double M, int R,
     finish_grads(k, gS, gs2, dS, u, out, sh);
 }
 
+// gS_j = (R q_j - sum_r p_jr^2) / 2, a workgroup per row of p (k x R): with many
+// right-hand sides one workgroup for the whole of fs_finish read p row by row
+// on one CU (k = 150, R = 2000: 195 us; this kernel and the finish: 8 us).
+__global__ __launch_bounds__(FT) void fs_rows_kernel(int R, const double* __restrict__ q,
+                                                     const double* __restrict__ p,
+                                                     double* __restrict__ gS) {
+    __shared__ double sh[FT / 64];
+    const int j = blockIdx.x;
+    double pp = 0.0;
+    for (int r = threadIdx.x; r < R; r += FT) pp += p[(size_t)j * R + r] * p[(size_t)j * R + r];
+    pp = block_sum(pp, sh);
+    if (threadIdx.x == 0) gS[j] = 0.5 * ((double)R * q[j] - pp);
+}
+
 // Function-space finish over R right-hand sides.  Inputs: q_j =
-// |L^-1 phi_j|^2, p = Phi^T a (k x R, row-major, leading dimension R),
-// ya = sum_r y_r^T a_r, aa = |a|_F^2, logdet_half = sum log L_ii.
+// |L^-1 phi_j|^2, p = Phi^T a (k x R, row-major, leading dimension R; NULL:
+// gS is there already), ya = sum_r y_r^T a_r, aa = |a|_F^2, logdet_half =
+// sum log L_ii.
 __global__ __launch_bounds__(FT) void fs_finish_kernel(int k, double M, int R,
                                                        const double* __restrict__ q,
                                                        const double* __restrict__ p,
@@ -305,6 +320,7 @@ __global__ __launch_bounds__(FT) void fs_finish_kernel(int k, double M, int R,
     double sq = 0.0;
     for (int j = threadIdx.x; j < k; j += FT) {
         sq += S[j] * q[j];
+        if (p == nullptr) continue;
         double pp = 0.0;
         for (int r = 0; r < R; ++r) pp += p[(size_t)j * R + r] * p[(size_t)j * R + r];
         gS[j] = 0.5 * (Rd * q[j] - pp);
@@ -468,9 +484,11 @@ extern "C" int rvgp_fs_finish(int k, double M, int nrhs, const double* q, const 
                               const double* S, const double* dS, const double* s2, const double* u,
                               double* gS, double* out, void* stream) {
     RVGP_CHECK_ARG(k >= 1 && nrhs >= 1, "rvgp_fs_finish: bad sizes");
-    hipLaunchKernelGGL(fs_finish_kernel, dim3(1), dim3(FT), 0, as_stream(stream), k, M, nrhs, q, p, ya,
-                       aa,
-                       logdet_half, S, dS, s2, u, gS, out);
+    const bool rows = nrhs >= 16;  // fewer: the second launch costs more than the loop
+    if (rows)
+        hipLaunchKernelGGL(fs_rows_kernel, dim3(k), dim3(FT), 0, as_stream(stream), nrhs, q, p, gS);
+    hipLaunchKernelGGL(fs_finish_kernel, dim3(1), dim3(FT), 0, as_stream(stream), k, M, nrhs, q,
+                       rows ? nullptr : p, ya, aa, logdet_half, S, dS, s2, u, gS, out);
     RVGP_LAUNCH_CHECK();
     return RVGP_OK;
 }

@@ -166,10 +166,16 @@ class GPREngine:
         if self.form == "function":
             if not self.normal:
                 self.K = torch.empty((self.M, self.M), **f64)
+                # [y | Phi], solved against the factor in one go
+                self.rows = torch.cat([self.y, self.Phi], 1).contiguous()
+                self.Z = torch.empty_like(self.rows)
+                self.colsq = torch.empty(self.R + self.k, **f64)
+                self.ones = torch.ones(self.R, **f64)
+                self._cs_ws = torch.empty(
+                    _lib.lib().rvgp_colsumsq_ws_bytes(self.M, self.R + self.k) // 8 + 1, **f64)
             if not self.coef:
                 self.a = torch.empty((self.M, self.R), **f64)
-                self.Z = torch.empty_like(self.Phi)
-            self.q = torch.empty(self.k, **f64)
+            self.q = torch.empty(self.k, **f64) if self.normal else self.colsq[self.R:]
             self.logdet = torch.empty(1, **f64)
 
     def _scalars(self):
@@ -332,15 +338,15 @@ class GPREngine:
             p = dense.gemm(self.Phi, self.a, transA=True)  # (k, R)
         else:
             self._factor()
-            # a = K_y^-1 y: L^-1 y first (ya = |L^-1 y|^2), then L^-T
-            self.a.copy_(self.y)
-            dense.trsm(self.K, self.a)
-            self._dot(self.a, self.a, self.ya)
+            # L^-1 [y | Phi]: its column norms are ya = |L^-1 y|^2 and q; then
+            # a = K_y^-1 y = L^-T L^-1 y
+            self.Z.copy_(self.rows)
+            dense.trsm(self.K, self.Z)
+            self._colsumsq(self.Z, self.colsq)
+            self._dot(self.colsq[:self.R], self.ones, self.ya)
+            self.a.copy_(self.Z[:, :self.R])
             dense.trsm(self.K, self.a, trans=True)
             self._dot(self.a, self.a, self.aa)
-            self.Z.copy_(self.Phi)
-            dense.trsm(self.K, self.Z)
-            self._colsumsq(self.Z, self.q)
             p = dense.gemm(self.Phi, self.a, transA=True)  # (k, R)
         if self.normal:
             _lib.call("rvgp_lemma_terms", self.k, float(self.M), _lib.ptr(self.S),
