@@ -220,6 +220,31 @@ int rvgp_bsr_spmm_f16(int nb, int b, const int* rowptr, const int* cols, const f
 int rvgp_frame_apply(int mode, int F, int n, int D, int d, const double* T, int ldt,
                      const double* in, double* out, void* stream);
 
+/* One Chebyshev series on a block-CSR operator (block size b = 1, 2, 3; FP64):
+ * out = sum_{j < terms} C_j o T_j with T_0 in t0, T_1 = (a A + shift) T_0 / 2,
+ * T_j = (a A + shift) T_{j-1} - T_{j-2}; t0 and t1 are overwritten.  Blocks are
+ * nb*b rows of ld <= 64 doubles (even, 16-byte aligned, unused columns zero);
+ * coef (terms, ld) on the device, a coefficient per term and column; active[j]
+ * (HOST, non-increasing): the columns with coefficients from term j on. */
+typedef struct {
+    int nb, b;
+    const int* rowptr;
+    const int* cols;
+    const double* vals;
+    double* t0;
+    double* t1;
+    double* out;
+    const double* coef;
+    int ld, terms;
+    const int* active;
+    double a, shift;
+} rvgp_series;
+
+/* The heat kernels of smoothing.py:13-15 (expm(-t L) x) and of the vector
+ * diffusion of smoothing.py:37-64, which needs one per Laplacian: one launch
+ * per term, shared by two one-field series. */
+int rvgp_cheb_series(int nops, const rvgp_series* ops, void* stream);
+
 /* out (rows, d) with row stride ldo, in place:
  *   out_i <- out_i * a_i / (b_i * |out_i|)   (a, b with strides lda, ldb). */
 int rvgp_diffusion_normalise(size_t rows, int d, double* out, int ldo, const double* a, int lda,

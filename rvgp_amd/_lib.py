@@ -21,6 +21,13 @@ D = ctypes.c_double
 F = ctypes.c_float
 S = ctypes.c_size_t
 
+
+class Series(ctypes.Structure):
+    """rvgp_series of include/rvgp.h."""
+    _fields_ = [("nb", I), ("b", I), ("rowptr", P), ("cols", P), ("vals", P), ("t0", P), ("t1", P),
+                ("out", P), ("coef", P), ("ld", I), ("terms", I), ("active", P), ("a", D), ("shift", D)]
+
+
 # name -> (restype, argtypes); mirrors include/rvgp.h
 SIGNATURES = {
     "rvgp_version": (I, []),
@@ -51,6 +58,7 @@ SIGNATURES = {
     "rvgp_chol_logdet": (I, [I, I, P, I, P, P]),
     "rvgp_frame_apply": (I, [I, I, I, I, I, P, I, P, P, P]),
     "rvgp_diffusion_normalise": (I, [S, I, P, I, P, I, P, I, P]),
+    "rvgp_cheb_series": (I, [I, P, P]),
     "rvgp_phi_rows": (I, [I, I, I, I, I, P, I, I, P, I, P, P, I, P]),
     "rvgp_gemm_sym": (I, [I, I, I, P, I, P, I, P, I, I, P, S, P]),
     "rvgp_syev_ws_bytes": (S, [I]),

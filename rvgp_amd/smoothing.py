@@ -10,11 +10,12 @@ the Gershgorin bound):
     c_j = (2 - [j = 0]) (-1)^j I_j(t ub / 2) exp(-t ub / 2),
 
 with I_j the modified Bessel functions (scipy.special.ive on the host, a
-handful of scalars).  The three-term recurrence runs as fused BSR SpMMs that
-also accumulate c_j T_j X into the result (rvgp_bsr_spmm's `acc` epilogue),
-so the operator is applied once per term with no extra passes.  The series is
-truncated when the remaining coefficients sum below 1e-17 of the first.
+handful of scalars).  The three-term recurrence and the sum run as one launch a
+term (rvgp_cheb_series).  The series is truncated when the remaining
+coefficients sum below 1e-17 of the first.
 """
+import ctypes
+
 import numpy as np
 import scipy.special
 import torch
@@ -37,6 +38,57 @@ def cheb_coeffs(t, ub, rtol=1e-17, max_terms=200000):
     return c[:max(J, 2)]
 
 
+SERIES_COLUMNS = 64  # most columns of one rvgp_cheb_series block
+
+
+class _Series:
+    """exp(-t (A - shift)) X for an FP64 X (rows, r <= 64) as an rvgp_series:
+    columns ordered by the length of their series, the row stride even."""
+
+    def __init__(self, A, X, ts, ub, shift):
+        r = X.shape[1]
+        ubs = ub - shift
+        made = {t: cheb_coeffs(t, ubs) for t in set(ts)}
+        cs = [made[ts[c if len(ts) > 1 else 0]] for c in range(r)]
+        order = sorted(range(r), key=lambda c: -len(cs[c]))
+        J, ld = len(cs[order[0]]), r + r % 2
+        C = np.zeros((J, ld))
+        for at, c in enumerate(order):
+            C[:len(cs[c]), at] = cs[c]
+        self.r, self.order = r, None if order == list(range(r)) else order
+        f64 = dict(dtype=torch.float64, device=X.device)
+        self.t0 = torch.zeros((X.shape[0], ld), **f64)
+        self.t0[:, :r] = X if self.order is None else X[:, order]
+        self.t1, self.out = torch.empty_like(self.t0), torch.empty_like(self.t0)
+        self.coef = torch.as_tensor(C, device=X.device)
+        lengths = np.array([len(cs[c]) for c in order])
+        self.active = np.ascontiguousarray((lengths[None, :] > np.arange(J)[:, None]).sum(1), np.int32)
+        # T_1 = (2/ubs)(A - shift) X - X ; T_j = (4/ubs)(A - shift) T_{j-1} - 2 T_{j-1} - T_{j-2}
+        self.op = _lib.Series(A.nb, A.b, *(t.data_ptr() for t in (A.rowptr, A.cols, A.vals64, self.t0,
+                                                                  self.t1, self.out, self.coef)),
+                              ld, J, self.active.ctypes.data, 4.0 / ubs, -2.0 - 4.0 * shift / ubs)
+
+    def result(self):
+        if self.order is None:
+            return self.out if self.r == self.out.shape[1] else self.out[:, :self.r]
+        back = np.empty(self.r, np.int64)
+        back[self.order] = np.arange(self.r)
+        return self.out[:, torch.as_tensor(back, device=self.out.device)]
+
+
+def _run_series(*series):
+    ops = (_lib.Series * len(series))(*(s.op for s in series))
+    _lib.call("rvgp_cheb_series", len(series), ctypes.byref(ops), _lib.stream())
+
+
+def _times(t, columns):
+    """Diffusion times as a list: one, or one per column."""
+    ts = [float(x) for x in np.atleast_1d(np.asarray(t, dtype=np.float64))]
+    if len(ts) > 1 and len(ts) != columns:
+        raise ValueError(f"{len(ts)} diffusion times for {columns} columns")
+    return ts
+
+
 def expm_multiply(A: BSR, X, t, ub=None, shift=0.0):
     """exp(-t (A - shift I)) X for a PSD BSR operator A (X: (rows,) or
     (rows, r)); shift must not exceed A's smallest eigenvalue.  t is a
@@ -51,65 +103,39 @@ def expm_multiply(A: BSR, X, t, ub=None, shift=0.0):
     exp(-t shift) is the caller's (normalised diffusion divides it out)."""
     if ub is None:
         ub = A.spectral_upper_bound() * 1.0001 + 1e-12
-    shift = float(shift)
-    if shift > 0.0:
-        # the series of exp(-t lambda') on [0, ub - shift] in lambda' = lambda - shift
-        return _expm_multiply_shifted(A, X, t, ub, shift)
+    shift = max(float(shift), 0.0)
     X2 = X.reshape(-1, 1) if X.dim() == 1 else X
-    ts = np.atleast_1d(np.asarray(t, dtype=np.float64))
-    if ts.size > 1:
-        if ts.size != X2.shape[1]:
-            raise ValueError(f"{ts.size} diffusion times for {X2.shape[1]} columns")
-        cs = [cheb_coeffs(tc, ub) for tc in ts]
-        C = np.zeros((max(len(c) for c in cs), ts.size))
-        for col, c in enumerate(cs):
-            C[:len(c), col] = c
-        Cd = torch.as_tensor(C, dtype=X2.dtype, device=X2.device)
-        out = X2 * Cd[0]
-        T1 = spmm(A, X2, alpha=2.0 / ub, beta=-1.0)
-        out.addcmul_(T1, Cd[1])
-        prev, cur = X2.clone(), T1
-        for j in range(2, C.shape[0]):
-            spmm(A, cur, Y=prev, alpha=4.0 / ub, beta=-2.0, Z=prev, gamma=-1.0)
-            out.addcmul_(prev, Cd[j])
-            prev, cur = cur, prev
-        return out.reshape(X.shape)
-    c = cheb_coeffs(float(ts[0]), ub)
-    out = X2 * float(c[0])
-    if len(c) > 1:
-        # T_1 = (2/ub) A X - X
-        T1 = spmm(A, X2, alpha=2.0 / ub, beta=-1.0, acc=out, delta=float(c[1]))
-        prev, cur = X2.clone(), T1
-        for j in range(2, len(c)):
-            # T_j = (4/ub) A T_{j-1} - 2 T_{j-1} - T_{j-2}, written over T_{j-2}
-            spmm(A, cur, Y=prev, alpha=4.0 / ub, beta=-2.0, Z=prev, gamma=-1.0, acc=out,
-                 delta=float(c[j]))
-            prev, cur = cur, prev
+    ts = _times(t, X2.shape[1])
+    if X2.dtype != torch.float64:
+        return _expm_spmm(A, X2, ts, ub, shift).reshape(X.shape)
+    parts = []
+    for c0 in range(0, X2.shape[1], SERIES_COLUMNS):
+        c1 = min(c0 + SERIES_COLUMNS, X2.shape[1])
+        s = _Series(A, X2[:, c0:c1], ts[c0:c1] if len(ts) > 1 else ts, ub, shift)
+        _run_series(s)
+        parts.append(s.result())
+    out = parts[0] if len(parts) == 1 else torch.cat(parts, 1)
     return out.reshape(X.shape)
 
 
-def _expm_multiply_shifted(A, X, t, ub, shift):
+def _expm_spmm(A, X2, ts, ub, shift):
+    """The series by block SpMMs, for blocks of other types than FP64."""
     ubs = ub - shift
-    X2 = X.reshape(-1, 1) if X.dim() == 1 else X
-    ts = np.atleast_1d(np.asarray(t, dtype=np.float64))
     cs = [cheb_coeffs(tc, ubs) for tc in ts]
     C = np.zeros((max(len(c) for c in cs), X2.shape[1]))
     for col in range(X2.shape[1]):
-        c = cs[col if ts.size > 1 else 0]
+        c = cs[col if len(ts) > 1 else 0]
         C[:len(c), col] = c
     Cd = torch.as_tensor(C, dtype=X2.dtype, device=X2.device)
-    # T_1 = (2/ubs)(A - shift) X - X ; T_j = (4/ubs)(A - shift) T_{j-1} - 2 T_{j-1} - T_{j-2}
     out = X2 * Cd[0]
-    if C.shape[0] > 1:
-        T1 = spmm(A, X2, alpha=2.0 / ubs, beta=-1.0 - 2.0 * shift / ubs)
-        out.addcmul_(T1, Cd[1])
-        prev, cur = X2.clone(), T1
-        for j in range(2, C.shape[0]):
-            spmm(A, cur, Y=prev, alpha=4.0 / ubs, beta=-2.0 - 4.0 * shift / ubs, Z=prev,
-                 gamma=-1.0)
-            out.addcmul_(prev, Cd[j])
-            prev, cur = cur, prev
-    return out.reshape(X.shape)
+    T1 = spmm(A, X2, alpha=2.0 / ubs, beta=-1.0 - 2.0 * shift / ubs)
+    out.addcmul_(T1, Cd[1])
+    prev, cur = X2.clone(), T1
+    for j in range(2, C.shape[0]):
+        spmm(A, cur, Y=prev, alpha=4.0 / ubs, beta=-2.0 - 4.0 * shift / ubs, Z=prev, gamma=-1.0)
+        out.addcmul_(prev, Cd[j])
+        prev, cur = cur, prev
+    return out
 
 
 def lambda_min_lower(A: BSR, evals=None, residual=None):
@@ -142,17 +168,27 @@ def vector_diffusion_device(c, t, Lc: BSR, L: BSR, lc_min=0.0):
     per_field = ts.size > 1
     if per_field and ts.size != F:
         raise ValueError(f"{ts.size} diffusion times for {F} fields")
+    tl = [float(x) for x in ts]
     # connection diffusion of every field: columns = fields
     Xc = C.reshape(F, n * d).T.contiguous()
-    out = expm_multiply(Lc, Xc, ts if per_field else float(ts[0]),
-                        shift=lc_min).T.reshape(F, n, d).contiguous()
     # scalar diffusions exp(-tL)|x| and exp(-tL)1 share one multi-column pass
     # (one column of ones per distinct time)
     n1 = F if per_field else 1
     xs = torch.empty((n, F + n1), dtype=torch.float64, device=c.device)
     xs[:, :F] = torch.linalg.vector_norm(C, dim=2).T
     xs[:, F:] = 1.0
-    sd = expm_multiply(L, xs, np.concatenate([ts, ts]) if per_field else float(ts[0]))
+    if F == 1:
+        # one field: small operators are bound by the launches, which the two
+        # series share
+        both = [_Series(A, X, tl, A.spectral_upper_bound() * 1.0001 + 1e-12, sh)
+                for A, X, sh in ((Lc, Xc, max(float(lc_min), 0.0)), (L, xs, 0.0))]
+        _run_series(*both)
+        out, sd = (s.result() for s in both)
+    else:
+        out = expm_multiply(Lc, Xc, tl, shift=lc_min)
+        sd = expm_multiply(L, xs, tl + tl if per_field else tl)
+    out = out.T.reshape(F, n, d).contiguous()
+    sd = sd.contiguous()
     for f in range(F):
         one = F + (f if per_field else 0)
         _lib.call("rvgp_diffusion_normalise", n, d, _lib.ptr(out[f]), d, _lib.ptr(sd[:, f:]),
