@@ -157,6 +157,9 @@ class data:
         self._Sigma = Sigma
         self._R = conn["R"]
         self._Lb, self._Lcb = Lb, Lcb
+        # the same operators in the eigensolver's numbering, for products with
+        # fields (their gathers then stay within an XCD's L2)
+        self._Lb_e, self._Lcb_e, self._perm = Lb_e, Lcb_e, perm
         self._evals_L = wL
         self._evecs_L = VL
         self._evals_Lc = wLc
@@ -330,8 +333,9 @@ class data:
                                                  self._evals_L, self._evecs_L)
         elif method == "matrix_exp":
             st = self.eig_stats["Lc"]
-            lc_min = lambda_min_lower(self._Lcb, float(self._evals_Lc[0].item()), st["residual"])
-            c = vector_diffusion_device(c, t, self._Lcb, self._Lb, lc_min=lc_min)
+            lc_min = lambda_min_lower(self._Lcb_e, float(self._evals_Lc[0].item()), st["residual"])
+            c = vector_diffusion_device(c, t, self._Lcb_e, self._Lb_e, lc_min=lc_min,
+                                        perm=self._perm)
         else:
             raise NotImplementedError
         self.vectors = self._frame(1, c, self._X.shape[1])

@@ -152,7 +152,7 @@ def lambda_min_lower(A: BSR, evals=None, residual=None):
     return max(0.0, theta - 2.0 * res - 1e-12 * scale)
 
 
-def vector_diffusion_device(c, t, Lc: BSR, L: BSR, lc_min=0.0):
+def vector_diffusion_device(c, t, Lc: BSR, L: BSR, lc_min=0.0, perm=None):
     """smoothing.py:37-64 (method="matrix_exp", normalise=True) on device.
 
     c: (n, d) local-frame coefficients, or (F, n, d) for F fields at once;
@@ -160,9 +160,12 @@ def vector_diffusion_device(c, t, Lc: BSR, L: BSR, lc_min=0.0):
     of Lc's smallest eigenvalue; the connection diffusion runs shifted by it
     (exp(-t lc_min) is common to every node and cancels in the
     normalisation), which keeps the smoothed directions accurate however
-    small exp(-t Lc) c is."""
+    small exp(-t Lc) c is.  perm: Lc and L are renumbered, perm[new] = old node;
+    c and the result are not."""
     batched = c.dim() == 3
     C = c if batched else c.unsqueeze(0)
+    if perm is not None:
+        C = C.index_select(1, perm)
     F, n, d = C.shape
     ts = np.atleast_1d(np.asarray(t, dtype=np.float64))
     per_field = ts.size > 1
@@ -193,6 +196,8 @@ def vector_diffusion_device(c, t, Lc: BSR, L: BSR, lc_min=0.0):
         one = F + (f if per_field else 0)
         _lib.call("rvgp_diffusion_normalise", n, d, _lib.ptr(out[f]), d, _lib.ptr(sd[:, f:]),
                   F + n1, _lib.ptr(sd[:, one:]), F + n1, _lib.stream())
+    if perm is not None:
+        out = torch.empty_like(out).index_copy_(1, perm, out)
     return out if batched else out[0]
 
 

@@ -27,10 +27,14 @@ class BSR:
 
     def gershgorin_bound(self):
         """max_i sum_j |A_ij| >= lambda_max (host scalar): the row sums are
-        |A| 1, one narrow block SpMM with the absolute values."""
+        |A| 1, one narrow block SpMM with the absolute values; cached on the
+        operator."""
+        if getattr(self, "_gb", None) is not None:
+            return self._gb
         absA = BSR(self.rowptr, self.cols, self.vals64.abs(), None, self.b)
         ones = torch.ones(self.shape[0], dtype=torch.float64, device=self.vals64.device)
-        return float(spmm(absA, ones).max().item())
+        self._gb = float(spmm(absA, ones).max().item())
+        return self._gb
 
     def spectral_upper_bound(self, steps=40, seed=20111):
         """Upper bound of lambda_max for the Chebyshev filters and the heat
