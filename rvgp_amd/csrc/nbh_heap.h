@@ -13,164 +13,180 @@ namespace rvgp {
 enum : int { kScanned = 0, kNotInHeap = 1, kInHeap = 2 };
 constexpr int kMaxRank = 32;
 
-// 32 bytes, aligned: a node never straddles two cache lines
-struct __align__(32) HNode {
+// A heap node; HNode's links index a pool of any size, LNode's (24 bytes, for
+// pools in LDS) one below 32768.  `last` is the rightmost child.
+template <class Idx>
+struct __align__(8) NodeOf {
     double val;
-    int gidx, parent, left, right, children;
+    int gidx;
     short rank, state;
+    Idx parent, left, right, children, last;
+};
+using HNode = NodeOf<int>;
+
+// LNode has no state: the wave's search keeps it in a mask.
+struct __align__(8) LNode {
+    double val;
+    int gidx;
+    short rank, parent, left, right, children, last;
 };
 
 // The root list is the sibling list holding min_node.  Its two ends are kept
-// in head / tail, so appending a root and finding the leftmost root are O(1)
-// instead of walks over the list: the reference walks it (pyx:526-536,
-// 642-660), but the walks only locate its ends, and the list itself -- every
-// link, every order -- is the same.
-struct Heap {
-    HNode* N;
+// in head / tail, and every node knows its rightmost child, so appending a
+// root or a child and finding the leftmost root are O(1) instead of walks
+// over the list: the reference walks it (pyx:526-536, 642-660), but the walks
+// only locate its ends, and the list itself -- every link, every order -- is
+// the same.
+template <class Node>
+struct HeapOf {
+    Node* N;
     int* roots;
     int min_node;
     int head, tail;
 };
+using Heap = HeapOf<HNode>;
 
-__host__ __device__ inline int rightmost_sibling(HNode* N, int a) {
-    while (N[a].right != -1) a = N[a].right;
-    return a;
-}
-
-__host__ __device__ inline int leftmost_sibling(HNode* N, int a) {
+template <class Node>
+__host__ __device__ inline int leftmost_sibling(const Node* N, int a) {
     while (N[a].left != -1) a = N[a].left;
     return a;
 }
 
-__host__ __device__ inline void add_sibling(HNode* N, int a, int s) {  // pyx:526-536
-    int t = rightmost_sibling(N, a);
-    N[t].right = s;
-    N[s].left = t;
-    N[s].right = -1;
-    N[s].parent = N[a].parent;
-    if (N[s].parent != -1) N[N[s].parent].rank += 1;
+// A root leaves the root list (pyx:542-560 where the parent is -1); its own
+// links are the caller's to set.
+template <class Node>
+__host__ __device__ inline void root_unlink(HeapOf<Node>& h, int a, int left, int right) {
+    if (a == h.head) h.head = right;
+    if (a == h.tail) h.tail = left;
+    if (left != -1) h.N[left].right = right;
+    if (right != -1) h.N[right].left = left;
 }
 
-__host__ __device__ inline void add_child(HNode* N, int a, int c) {  // pyx:507-520
-    N[c].parent = a;
-    if (N[a].children != -1) {
-        add_sibling(N, N[a].children, c);
-    } else {
-        N[a].children = c;
-        N[c].right = -1;
-        N[c].left = -1;
-        N[a].rank = 1;
-    }
-}
-
-__host__ __device__ inline void node_remove(Heap& h, int a) {  // pyx:542-560
-    HNode* N = h.N;
-    int p = N[a].parent;
-    if (p == -1) {  // a root: keep the list's ends
-        if (a == h.head) h.head = N[a].right;
-        if (a == h.tail) h.tail = N[a].left;
-    } else {
-        N[p].rank -= 1;
-        if (N[a].left != -1) N[p].children = N[a].left;
-        else if (N[a].right != -1) N[p].children = N[a].right;
-        else N[p].children = -1;
-    }
-    if (N[a].left != -1) N[N[a].left].right = N[a].right;
-    if (N[a].right != -1) N[N[a].right].left = N[a].left;
-    N[a].left = -1;
-    N[a].right = -1;
+// A child leaves its parent (pyx:542-560).
+template <class Node>
+__host__ __device__ inline void child_remove(HeapOf<Node>& h, int a) {
+    Node* N = h.N;
+    const int p = N[a].parent, l = N[a].left, r = N[a].right;
+    N[p].rank -= 1;
+    N[p].children = l != -1 ? l : r;
+    if (N[p].last == a) N[p].last = l;
+    if (l != -1) N[l].right = r;
+    if (r != -1) N[r].left = l;
     N[a].parent = -1;
 }
 
 // add_sibling(min_node, s) for the root list (pyx:526-536): s goes after
 // the rightmost root; a root's parent is -1, so no rank changes.
-__host__ __device__ inline void root_append(Heap& h, int s) {
-    HNode* N = h.N;
+template <class Node>
+__host__ __device__ inline void root_append(HeapOf<Node>& h, int s) {
+    Node* N = h.N;
     N[h.tail].right = s;
     N[s].left = h.tail;
     N[s].right = -1;
-    N[s].parent = -1;
     h.tail = s;
 }
 
-__host__ __device__ inline void insert_node(Heap& h, int a) {  // pyx:579-589
+// pyx:579-589, of a node without parent
+template <class Node>
+__host__ __device__ inline void insert_node(HeapOf<Node>& h, int a) {
     if (h.min_node != -1) {
         root_append(h, a);
         if (h.N[a].val < h.N[h.min_node].val) h.min_node = a;
     } else {
+        h.N[a].left = h.N[a].right = -1;
         h.min_node = a;
         h.head = h.tail = a;
     }
 }
 
-__host__ __device__ inline void decrease_val(Heap& h, int a, double v) {  // pyx:595-608
-    HNode* N = h.N;
+template <class Node>
+__host__ __device__ inline void decrease_val(HeapOf<Node>& h, int a, double v) {  // pyx:595-608
+    Node* N = h.N;
     N[a].val = v;
     if (N[a].parent != -1 && N[N[a].parent].val >= v) {
-        node_remove(h, a);
+        child_remove(h, a);
         insert_node(h, a);
-    } else if (N[h.min_node].val > N[a].val) {
+    } else if (N[h.min_node].val > v) {
         h.min_node = a;
     }
 }
 
-// pyx:614-636 (tail recursion as a loop).  Returns false on rank overflow.
-__host__ __device__ inline bool heap_link(Heap& h, int a) {
-    HNode* N = h.N;
-    for (;;) {
-        int r = N[a].rank;
-        if (r >= kMaxRank) return false;
-        if (h.roots[r] == -1) {
-            h.roots[r] = a;
-            return true;
-        }
-        int ln = h.roots[r];
-        h.roots[r] = -1;
-        if (N[a].val < N[ln].val || a == h.min_node) {
-            node_remove(h, ln);
-            add_child(N, a, ln);
-        } else {
-            node_remove(h, a);
-            add_child(N, ln, a);
-            a = ln;
-        }
-    }
-}
-
-// pyx:642-690.  The reference clears roots_by_rank[0..100); ranks here are
-// bounded by kMaxRank (checked), so clearing [0, kMaxRank) is equivalent.
-__host__ __device__ inline int remove_min(Heap& h, bool& ok) {
-    HNode* N = h.N;
-    int m = h.min_node, t, tr;
+// pyx:642-690 with the linking of pyx:614-636.  The reference clears
+// roots_by_rank[0..100); ranks here are bounded by kMaxRank (checked), so
+// clearing [0, kMaxRank) is equivalent.  The children of the minimum become
+// roots as one splice of their list: its order is the one that appending them
+// from the leftmost on gives.  Two linked roots have the same rank r, and the
+// parent's is r + 1 after it, so ranks and values of the running root stay in
+// registers.
+template <class Node>
+__host__ __device__ inline int remove_min(HeapOf<Node>& h, bool& ok) {
+    Node* N = h.N;
+    const int m = h.min_node;
     if (N[m].children != -1) {
-        t = leftmost_sibling(N, N[m].children);
-        while (t != -1) {
-            tr = N[t].right;
-            node_remove(h, t);
-            root_append(h, t);  // add_sibling(m, t): m is a root
-            t = tr;
-        }
+        const int first = leftmost_sibling(N, N[m].children), last = N[m].last;
+        for (int c = first; c != -1; c = N[c].right) N[c].parent = -1;
+        N[h.tail].right = first;
+        N[first].left = h.tail;
+        h.tail = last;
         N[m].children = -1;
+        N[m].rank = 0;
     }
-    t = h.head;  // leftmost_sibling(m)
+    int t = h.head;  // leftmost_sibling(m)
     if (t == m) {
-        if (N[m].right != -1) {
-            t = N[m].right;
-        } else {
+        t = N[m].right;
+        if (t == -1) {
             h.min_node = -1;
             h.head = h.tail = -1;
             return m;
         }
     }
-    node_remove(h, m);
-    h.min_node = t;
+    root_unlink(h, m, N[m].left, N[m].right);
+    int mn = t;
+    double mv = N[t].val;
     for (int i = 0; i < kMaxRank; ++i) h.roots[i] = -1;
     while (t != -1) {
-        if (N[t].val < N[h.min_node].val) h.min_node = t;
-        tr = N[t].right;
-        if (!heap_link(h, t)) { ok = false; return m; }
+        int a = t, r = N[t].rank;
+        double va = N[t].val;
+        const int tr = N[t].right;
+        if (va < mv) {
+            mn = t;
+            mv = va;
+        }
+        for (;;) {
+            if (r >= kMaxRank) {
+                ok = false;
+                h.min_node = mn;
+                return m;
+            }
+            const int ln = h.roots[r];
+            if (ln == -1) {
+                h.roots[r] = a;
+                break;
+            }
+            h.roots[r] = -1;
+            const double vl = N[ln].val;
+            const Node na = N[a], nl = N[ln];
+            const bool keep = va < vl || a == mn;
+            const int par = keep ? a : ln, ch = keep ? ln : a;
+            root_unlink(h, ch, keep ? nl.left : na.left, keep ? nl.right : na.right);
+            const int pc = keep ? na.children : nl.children, pl = keep ? na.last : nl.last;
+            N[ch].parent = par;  // add_child (pyx:507-520)
+            N[ch].right = -1;
+            if (pc != -1) {
+                N[pl].right = ch;
+                N[ch].left = pl;
+            } else {
+                N[par].children = ch;
+                N[ch].left = -1;
+            }
+            N[par].last = ch;
+            N[par].rank = ++r;
+            a = par;
+            va = keep ? va : vl;
+        }
         t = tr;
     }
+    h.min_node = mn;
     return m;
 }
 
@@ -210,7 +226,7 @@ __host__ __device__ inline bool nbh_search(const int* rowptr, const int* cols, c
         nd.gidx = g;
         nd.rank = 0;
         nd.state = kNotInHeap;
-        nd.parent = nd.left = nd.right = nd.children = -1;
+        nd.parent = nd.left = nd.right = nd.children = nd.last = -1;
         L.hposv[s] = (int)hp;
         tab[hp] = make_int2(g, s);
         return s;

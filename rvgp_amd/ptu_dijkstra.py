@@ -30,17 +30,15 @@ def _check_status(st):
 def geo_nbh_device(g, K, max_ws_bytes=16 << 30):
     """(n, K+1) int32 neighbourhoods in heap pop order (pyx:361-394).
 
-    One lane per source and every source in flight at once where the
-    workspace cap allows (~27 KB per lane in the first pass, whose node pool
-    holds what a search on a kNN graph touches; the few searches that
-    outgrow it are redone with the worst-case pool 1 + K * max_degree): the
-    heap walks are latency-bound, so the number of lanes in flight sets the
-    speed."""
+    A wavefront per source with its node pool in LDS; the few searches that
+    outgrow it are redone with the worst-case pool 1 + K * max_degree by up
+    to 2048 lanes in memory, so the workspace holds no more lanes than those
+    and room for the list of leftovers."""
     n = g.n
     pool = 1 + K * g.max_row()
     L = _lib.lib()
     per_lane = max(1, L.rvgp_geo_nbh_ws_bytes(n, 2, pool) - L.rvgp_geo_nbh_ws_bytes(n, 1, pool))
-    batch = int(max(1, min(n, max_ws_bytes // per_lane, 1 << 17)))
+    batch = int(max(1, min(n, max_ws_bytes // per_lane, 2048 + n // 1024)))
     ws_bytes = L.rvgp_geo_nbh_ws_bytes(n, batch, pool)
     dev = g.cols.device
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
