@@ -491,6 +491,17 @@ int rvgp_batch_step(int F, int k, int typ, const double* evals, double n_rows, c
                     int threads, int grid, double* ws, size_t ws_bytes, double* out, int* status,
                     void* stream);
 
+/* `steps` >= 1 of these steps one after another, the same results as as many
+ * calls.  The fits are independent: where a fit's factor fits in LDS (panel =
+ * 16, k <= 160) one launch does them all, a fit's G staying in registers;
+ * elsewhere it is a launch a step. */
+int rvgp_batch_steps(int F, int k, int typ, const double* evals, double n_rows, const double* G,
+                    const double* b, const double* yy, const double* M, const double* lower,
+                    double* u, const int* trainable, double* m1, double* m2, double* t,
+                    int do_adam, int steps, double lr, double b1, double b2, double eps, int panel,
+                    int threads, int grid, double* ws, size_t ws_bytes, double* out, int* status,
+                    void* stream);
+
 /* ---------------------------------------------------------------------
  * kernel='rbf' branch of RVGP.fit (RVGP/main.py:33-37): gpflow.kernels.RBF
  * on evecs_L rows, the D vector components as D output columns of one GPR.

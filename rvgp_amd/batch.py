@@ -8,10 +8,10 @@ subset, of any size, and its own hyperparameters -- are fitted together:
     (rvgp_batch_gram: G_f = Phi_f^T Phi_f over the fit's gathered intrinsic
     eigenvector rows, upper tiles on the matrix cores; rvgp_batch_rhs:
     b_f = Phi_f^T y_f and y_f^T y_f from the targets in the local frames);
-  * each optimiser step: ONE launch of rvgp_batch_step -- a persistent
-    kernel, one workgroup per fit, that forms A_f, factors it, evaluates the
-    NLML and its adjoint and applies Adam -- captured in a HIP graph and
-    replayed for every step.
+  * each optimiser step: a persistent kernel (rvgp_batch_steps), one workgroup
+    per fit, that forms A_f, factors it, evaluates the NLML and its adjoint and
+    applies Adam: many steps to a launch where the factor fits in LDS, else
+    one, captured in a HIP graph and replayed for every step.
 
 The NLML of each fit is the one of gp.GPREngine's weight-space form (exact for
 any subset size, identical to GPflow's function-space value).  Launch shapes
@@ -25,6 +25,14 @@ from .gp import inv_softplus, softplus
 from .kernels import ManifoldKernel
 
 GAUSSIAN_VARIANCE_LOWER_BOUND = 1e-6
+
+
+# Fits of up to this many eigenvectors keep their factor in LDS, and one launch
+# runs many steps of them (kLdsTiles in batch.hip): a launch a step, replayed
+# from a graph, took 70 us at k = 120, a step of many in one launch 45 us.
+# Enough steps to lose the launch, few enough that a launch stays near 2 ms.
+LDS_MAX_K = 160
+STEPS_PER_LAUNCH = 50
 
 
 class BatchedGPR:
@@ -124,14 +132,14 @@ class BatchedGPR:
         self.panel, self.threads = (int(panel), 512) if np.isscalar(panel) else map(int, panel)
 
     # ------------------------------------------------------------------ steps
-    def _step(self, do_adam, lr, b1=0.9, b2=0.999, eps=1e-8, panel=None):
+    def _step(self, do_adam, lr, b1=0.9, b2=0.999, eps=1e-8, panel=None, steps=1):
         nb, nt = (self.panel, self.threads) if panel is None else (
             (int(panel), 512) if np.isscalar(panel) else panel)
-        _lib.call("rvgp_batch_step", self.F, self.k, self.typ, _lib.ptr(self.evals), self.n_rows,
+        _lib.call("rvgp_batch_steps", self.F, self.k, self.typ, _lib.ptr(self.evals), self.n_rows,
                   _lib.ptr(self.G), _lib.ptr(self.b), _lib.ptr(self.yy), _lib.ptr(self.M),
                   _lib.ptr(self.lower), _lib.ptr(self.u), _lib.ptr(self.trainable),
-                  _lib.ptr(self.m1), _lib.ptr(self.m2), _lib.ptr(self.t), int(do_adam), float(lr),
-                  float(b1), float(b2), float(eps), int(nb), int(nt), self.grid,
+                  _lib.ptr(self.m1), _lib.ptr(self.m2), _lib.ptr(self.t), int(do_adam), int(steps),
+                  float(lr), float(b1), float(b2), float(eps), int(nb), int(nt), self.grid,
                   _lib.ptr(self.ws), self.ws_bytes, _lib.ptr(self.out), _lib.ptr(self.status),
                   _lib.stream())
 
@@ -155,7 +163,10 @@ class BatchedGPR:
         return g
 
     def fit(self, epochs=200, lr=0.05, use_graph=True):
-        if use_graph and epochs > 1:
+        if self.panel == 16 and self.k <= LDS_MAX_K:
+            for i in range(0, int(epochs), STEPS_PER_LAUNCH):
+                self._step(1, lr, steps=min(STEPS_PER_LAUNCH, int(epochs) - i))
+        elif use_graph and epochs > 1:
             g = self.capture_adam_step(lr)
             for _ in range(int(epochs)):
                 g.replay()

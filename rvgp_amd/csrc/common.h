@@ -67,6 +67,25 @@ __device__ __forceinline__ double bcast(double v, int l) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+// Sum over the wave by DPP row moves and broadcasts, in every lane.
+__device__ __forceinline__ double wave_sum_dpp(double v) {
+#define RVGP_STEP(CTRL, ROWS)                                                                     \
+    {                                                                                             \
+        const long long b = __double_as_longlong(v);                                             \
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);            \
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);    \
+        v += __longlong_as_double(((long long)hi << 32) | (unsigned)lo);                          \
+    }
+    RVGP_STEP(0x111, 0xf)
+    RVGP_STEP(0x112, 0xf)
+    RVGP_STEP(0x114, 0xf)
+    RVGP_STEP(0x118, 0xf)
+    RVGP_STEP(0x142, 0xa)
+    RVGP_STEP(0x143, 0xc)
+#undef RVGP_STEP
+    return bcast(v, 63);
+}
+
 // Direct squared distance with a fixed operation order:
 //   acc = fma(t_k, t_k, acc), t_k = a_k - b_k, k = 0..D-1.
 // The CPU oracle uses the same sequence, so results agree bit for bit.

@@ -1,6 +1,6 @@
 // Fibonacci-heap emulation of RVGP/lib/ptu_dijkstra.pyx:440-690 and the
 // per-source truncated Dijkstra of pyx:361-394, shared by the neighbourhood
-// kernel (nbh.hip, one lane per source) and the host build that runs the same
+// kernels (nbh.hip) and the host build that runs the same
 // code under AddressSanitizer / UndefinedBehaviorSanitizer
 // (tests/sanitize/nbh_host.hip).  Every function compiles for both sides.
 #ifndef RVGP_NBH_HEAP_H

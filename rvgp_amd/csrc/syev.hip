@@ -336,25 +336,6 @@ __device__ __forceinline__ double rcp_nr(double x) {
     return fma(fma(-x, r, 1.0), r, r);
 }
 
-// Sum over the wave by DPP row moves and broadcasts, in every lane.
-__device__ __forceinline__ double wave_sum_dpp(double v) {
-#define RVGP_STEP(CTRL, ROWS)                                                                     \
-    {                                                                                             \
-        const long long b = __double_as_longlong(v);                                             \
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);            \
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);    \
-        v += __longlong_as_double(((long long)hi << 32) | (unsigned)lo);                          \
-    }
-    RVGP_STEP(0x111, 0xf)
-    RVGP_STEP(0x112, 0xf)
-    RVGP_STEP(0x114, 0xf)
-    RVGP_STEP(0x118, 0xf)
-    RVGP_STEP(0x142, 0xa)
-    RVGP_STEP(0x143, 0xc)
-#undef RVGP_STEP
-    return bcast(v, 63);
-}
-
 // The whole tridiagonalisation of a matrix of n <= kSmallN in one workgroup,
 // the matrix in registers: wave v of NW owns the columns c = v (mod NW), lane
 // i of it the rows i + 64 k (k < R) of its C columns.  In step j every wave
