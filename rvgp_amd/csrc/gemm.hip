@@ -582,6 +582,13 @@ static int f32_big_slots() {
     return slots;
 }
 
+// K is split (as far as 1024 workgroups, 8 k-steps each) from where the small
+// kernel ends: one workgroup's k-loop over a tall Gram is a serial chain.  64 x
+// 64 from K = 1100: 128 us in one piece, 18 us in 17; K = 2000: 230 -> 18 us
+// (FP32 180 -> 19); 256 x 256, K = 2000: 344 -> 32 us.
+// Up to kSplitAlwaysK a caller's workspace of the unsplit product still does.
+constexpr int kSplitMinK = 1024, kSplitAlwaysK = 2048;
+
 // small: K <= 1024 and at most 64 tiles of the 128 x 128 kernel -- too few
 // workgroups to hide the k-loop latency, so one wave per 16 x 16 tile wins.
 static GemmPlan gemm_plan(int mode, int M, int N, int K, int BK, int split_k) {
@@ -598,7 +605,7 @@ static GemmPlan gemm_plan(int mode, int M, int N, int K, int BK, int split_k) {
     int split = split_k;
     if (split <= 0) {
         split = 1;
-        if (K >= 2048) {
+        if (K > kSplitMinK) {
             long s = (1024 + tiles - 1) / tiles;
             long smax = K / (8 * BK);
             if (s > smax) s = smax;
@@ -629,7 +636,10 @@ static int gemm_launch(int transA, int transB, int M, int N, int K, double alpha
     constexpr int MODE = MD == Mode::F64 ? RVGP_GEMM_F64
                          : MD == Mode::F32 ? RVGP_GEMM_F32
                          : MD == Mode::F32ACC64 ? RVGP_GEMM_F32_ACC64 : RVGP_GEMM_BF16;
-    const GemmPlan pl = gemm_plan(MODE, M, N, K, Tr<MD>::BK, split);
+    GemmPlan pl = gemm_plan(MODE, M, N, K, Tr<MD>::BK, split);
+    if (pl.split > 1 && split <= 0 && K < kSplitAlwaysK &&
+        (ws == nullptr || ws_bytes < sizeof(Acc) * (size_t)pl.split * M * N))
+        pl = gemm_plan(MODE, M, N, K, Tr<MD>::BK, 1);
     if constexpr (MD != Mode::BF16) {
         if (N == 1 && K <= 8192 && kscale == nullptr && !lower && !upper && split <= 1) {
             const int incx = transB ? 1 : ldb;
@@ -743,7 +753,10 @@ static int gram_f32_chunked(int M, int K, const float* A, int lda, const float* 
                    "rvgp_gemm_sym: bad sizes");
     if (M == 0) return RVGP_OK;
     hipStream_t s = as_stream(stream);
-    const GemmPlan pl = gram_f32_plan(M, K, split_k);
+    GemmPlan pl = gram_f32_plan(M, K, split_k);
+    if (split_k <= 0 && K < kSplitAlwaysK &&
+        (ws == nullptr || ws_bytes < sizeof(float) * (size_t)pl.split * M * M))
+        pl = gram_f32_plan(M, K, 1);
     const size_t need = sizeof(float) * (size_t)pl.split * M * M;
     RVGP_CHECK_ARG(ws != nullptr && ws_bytes >= need,
                    "rvgp_gemm_sym: the FP32 Gram needs %zu bytes of workspace", need);
