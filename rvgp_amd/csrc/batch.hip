@@ -632,23 +632,6 @@ __device__ __forceinline__ void wg_sum_n(double (&v)[N], double* sh) {
     }
 }
 
-// Lane l of each row of 16 lanes to all of that row, without a detour over
-// scalar registers (whose hazard costs as much as the product).  l is constant
-// at every use, so one case is left of the switch.
-__device__ __forceinline__ double row_bcast(double v, int l) {
-    switch (l) {
-#define RVGP_LANE(L)                                                             \
-    case L:                                                                      \
-        v = __builtin_amdgcn_update_dpp(v, v, 0x150 + L, 0xf, 0xf, true);        \
-        break;
-        RVGP_LANE(0) RVGP_LANE(1) RVGP_LANE(2) RVGP_LANE(3) RVGP_LANE(4) RVGP_LANE(5)
-        RVGP_LANE(6) RVGP_LANE(7) RVGP_LANE(8) RVGP_LANE(9) RVGP_LANE(10) RVGP_LANE(11)
-        RVGP_LANE(12) RVGP_LANE(13) RVGP_LANE(14) RVGP_LANE(15)
-#undef RVGP_LANE
-    }
-    return v;
-}
-
 // One wave factors the 16 x 16 tile T = L L^T: lane i holds row i (every
 // 16-lane row the same) and eliminates without square roots (a pivot's reciprocal by the hardware
 // estimate and one cubic step is all that the next column waits for); the

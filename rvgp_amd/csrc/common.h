@@ -67,6 +67,23 @@ __device__ __forceinline__ double bcast(double v, int l) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+// Lane l of each row of 16 lanes to all of that row, without a detour over
+// scalar registers (whose hazard costs as much as the product).  l is constant
+// at every use, so one case is left of the switch.
+__device__ __forceinline__ double row_bcast(double v, int l) {
+    switch (l) {
+#define RVGP_LANE(L)                                                             \
+    case L:                                                                      \
+        v = __builtin_amdgcn_update_dpp(v, v, 0x150 + L, 0xf, 0xf, true);        \
+        break;
+        RVGP_LANE(0) RVGP_LANE(1) RVGP_LANE(2) RVGP_LANE(3) RVGP_LANE(4) RVGP_LANE(5)
+        RVGP_LANE(6) RVGP_LANE(7) RVGP_LANE(8) RVGP_LANE(9) RVGP_LANE(10) RVGP_LANE(11)
+        RVGP_LANE(12) RVGP_LANE(13) RVGP_LANE(14) RVGP_LANE(15)
+#undef RVGP_LANE
+    }
+    return v;
+}
+
 // Sum over the wave by DPP row moves and broadcasts, in every lane.
 __device__ __forceinline__ double wave_sum_dpp(double v) {
 #define RVGP_STEP(CTRL, ROWS)                                                                     \
