@@ -250,84 +250,161 @@ __global__ void sym_count_kernel(const int* __restrict__ nbr, int n, int k, int*
     if (e < n) atomicAdd(&cnt[e], k + 1);
 }
 
-// Exclusive scan of cnt[0..n) into out[0..n], out[n] = total, in one block.
+// Exclusive scan of cnt[0..n) into out[0..n], out[n] = total: sums of chunks of
+// kScanChunk, then every chunk's block adds up the sums before its own and scans
+// it (n = 100000: 183 us in one workgroup -> 10 us).
 constexpr int kScanThreads = 1024;
-__global__ __launch_bounds__(kScanThreads) void scan_kernel(const int* __restrict__ cnt, int n,
-                                                            int* __restrict__ out) {
-    __shared__ int part[kScanThreads];
-    const int per = (n + kScanThreads - 1) / kScanThreads;
-    const int b = threadIdx.x * per;
-    const int e = min(n, b + per);
-    int s = 0;
-    for (int i = b; i < e; ++i) s += cnt[i];
-    part[threadIdx.x] = s;
+constexpr int kScanChunk = 4 * kScanThreads;
+
+__device__ __forceinline__ int block_sum_int(int v, int* sh) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     __syncthreads();
-    for (int o = 1; o < kScanThreads; o <<= 1) {
-        int v = (threadIdx.x >= o) ? part[threadIdx.x - o] : 0;
-        __syncthreads();
-        part[threadIdx.x] += v;
-        __syncthreads();
-    }
-    int run = part[threadIdx.x] - s;
-    for (int i = b; i < e; ++i) {
-        out[i] = run;
-        run += cnt[i];
-    }
-    if (threadIdx.x == kScanThreads - 1) out[n] = part[kScanThreads - 1];
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    int s = 0;
+    for (int i = 0; i < kScanThreads / 64; ++i) s += sh[i];
+    return s;
 }
 
+__global__ __launch_bounds__(kScanThreads) void scan_sums_kernel(const int* __restrict__ cnt, int n,
+                                                                 int* __restrict__ sums) {
+    __shared__ int sh[kScanThreads / 64];
+    int v = 0;
+    for (int q = 0; q < 4; ++q) {
+        const int i = blockIdx.x * kScanChunk + q * kScanThreads + threadIdx.x;
+        v += i < n ? cnt[i] : 0;
+    }
+    v = block_sum_int(v, sh);
+    if (threadIdx.x == 0) sums[blockIdx.x] = v;
+}
+
+__global__ __launch_bounds__(kScanThreads) void scan_kernel(const int* __restrict__ cnt, int n,
+                                                            const int* __restrict__ sums,
+                                                            int* __restrict__ out) {
+    __shared__ int sh[kScanThreads / 64];
+    int before = 0;
+    for (int i = threadIdx.x; i < (int)blockIdx.x; i += kScanThreads) before += sums[i];
+    before = block_sum_int(before, sh);
+    const int i0 = blockIdx.x * kScanChunk + 4 * threadIdx.x;
+    int c[4], mine = 0;
+    for (int q = 0; q < 4; ++q) {
+        c[q] = i0 + q < n ? cnt[i0 + q] : 0;
+        mine += c[q];
+    }
+    int incl = mine;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(incl, o, 64);
+        if ((threadIdx.x & 63) >= o) incl += v;
+    }
+    __syncthreads();
+    if ((threadIdx.x & 63) == 63) sh[threadIdx.x >> 6] = incl;
+    __syncthreads();
+    int run = before + incl - mine;
+    for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) run += sh[w];
+    for (int q = 0; q < 4; ++q) {
+        if (i0 + q < n) out[i0 + q] = run;
+        run += c[q];
+        if (i0 + q == n - 1) out[n] = run;
+    }
+}
+
+// A row's segment: itself, its k neighbours, then whoever has it as a neighbour
+// (in any order: the segments are sorted next).
 __global__ void sym_fill_kernel(const int* __restrict__ nbr, int n, int k,
                                 const int* __restrict__ start, int* __restrict__ cursor,
                                 int* __restrict__ tmp) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int pos = atomicAdd(&cursor[i], k + 1);
-    int* dst = tmp + start[i] + pos;
-    dst[0] = i;
-    for (int q = 0; q < k; ++q) {
-        const int j = nbr[(size_t)i * k + q];
-        if ((unsigned)j >= (unsigned)n) {
-            dst[1 + q] = i;
-            continue;
-        }
-        dst[1 + q] = j;
-        int pj = atomicAdd(&cursor[j], 1);
-        tmp[start[j] + pj] = i;
+    const unsigned e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= (unsigned)(n * k)) return;
+    const int i = (int)(e / (unsigned)k), q = (int)(e - (unsigned)i * k);
+    int* dst = tmp + start[i];
+    if (q == 0) dst[0] = i;
+    const int j = nbr[e];
+    if ((unsigned)j >= (unsigned)n) {
+        dst[1 + q] = i;
+        return;
     }
+    dst[1 + q] = j;
+    tmp[start[j] + k + 1 + atomicAdd(&cursor[j], 1)] = i;
 }
 
-// Sort each row segment in place (insertion sort; rows are short) and
-// count the unique entries.
-__global__ void sym_sort_kernel(const int* __restrict__ start, int n, int* __restrict__ tmp,
-                                int* __restrict__ ucnt) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// Sort each row segment in place and count its unique entries, a wave to a row:
+// an entry's place is the number of entries below it, equal ones in their
+// order.  Up to 64 entries (every row but hubs) are compared by readlane, up to
+// kSortLds from LDS; longer ones by insertion on one lane.  n = 100000, k = 20:
+// 459 us (insertion, a thread to a row) -> 57 us.
+constexpr int kSortWaves = 4, kSortLds = 1024;
+
+__global__ __launch_bounds__(64 * kSortWaves) void sym_sort_kernel(const int* __restrict__ start, int n,
+                                                                   int* __restrict__ tmp,
+                                                                   int* __restrict__ ucnt) {
+    __shared__ int lds[kSortWaves][kSortLds];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = blockIdx.x * kSortWaves + wv;
     if (i >= n) return;
     int* seg = tmp + start[i];
-    const int len = start[i + 1] - start[i];
-    for (int a = 1; a < len; ++a) {
-        int v = seg[a];
-        int p = a - 1;
-        while (p >= 0 && seg[p] > v) {
-            seg[p + 1] = seg[p];
-            --p;
-        }
-        seg[p + 1] = v;
-    }
+    const int len = __builtin_amdgcn_readfirstlane(start[i + 1] - start[i]);
     int u = 0;
-    for (int a = 0; a < len; ++a) u += (a == 0 || seg[a] != seg[a - 1]);
-    ucnt[i] = u;
+    if (len <= 64) {
+        const int v = lane < len ? seg[lane] : 0;
+        int rank = 0, twins = 0;
+        for (int b = 0; b < len; ++b) {
+            const int o = __builtin_amdgcn_readlane(v, b);
+            const bool twin = o == v && b < lane;
+            rank += o < v || twin;
+            twins += twin;
+        }
+        if (lane < len) seg[rank] = v;
+        u = __popcll(__ballot(lane < len && twins == 0));
+    } else if (len <= kSortLds) {
+        int* s = lds[wv];
+        for (int a = lane; a < len; a += 64) s[a] = seg[a];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        for (int a0 = 0; a0 < len; a0 += 64) {
+            const int a = a0 + lane, v = a < len ? s[a] : 0;
+            int rank = 0, twins = 0;
+            for (int b = 0; b < len; ++b) {
+                const int o = s[b];
+                const bool twin = o == v && b < a;
+                rank += o < v || twin;
+                twins += twin;
+            }
+            if (a < len) seg[rank] = v;
+            u += __popcll(__ballot(a < len && twins == 0));
+        }
+    } else if (lane == 0) {
+        for (int a = 1; a < len; ++a) {
+            const int v = seg[a];
+            int p = a - 1;
+            while (p >= 0 && seg[p] > v) {
+                seg[p + 1] = seg[p];
+                --p;
+            }
+            seg[p + 1] = v;
+        }
+        for (int a = 0; a < len; ++a) u += (a == 0 || seg[a] != seg[a - 1]);
+    }
+    if (lane == 0) ucnt[i] = u;
 }
 
-__global__ void sym_compact_kernel(const int* __restrict__ start, int n,
-                                   const int* __restrict__ tmp, const int* __restrict__ rowptr,
-                                   int* __restrict__ cols) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// A wave copies a row's unique entries.
+__global__ __launch_bounds__(64 * kSortWaves) void sym_compact_kernel(const int* __restrict__ start, int n,
+                                                                      const int* __restrict__ tmp,
+                                                                      const int* __restrict__ rowptr,
+                                                                      int* __restrict__ cols) {
+    const int lane = threadIdx.x & 63, i = blockIdx.x * kSortWaves + (threadIdx.x >> 6);
     if (i >= n) return;
     const int* seg = tmp + start[i];
     const int len = start[i + 1] - start[i];
     int o = rowptr[i];
-    for (int a = 0; a < len; ++a)
-        if (a == 0 || seg[a] != seg[a - 1]) cols[o++] = seg[a];
+    for (int a0 = 0; a0 < len; a0 += 64) {
+        const int a = a0 + lane;
+        const int v = a < len ? seg[a] : 0;
+        const bool first = a < len && (a == 0 || seg[a - 1] != v);
+        const unsigned long long m = __ballot(first);
+        if (first) cols[o + __popcll(m & ((1ull << lane) - 1))] = v;
+        o += __popcll(m);
+    }
 }
 
 template <int DMAX, int KM>
@@ -469,15 +546,24 @@ extern "C" int rvgp_graph_symmetrize(const int* nbr, int n, int k, int* rowptr, 
     const int T = 256;
     hipLaunchKernelGGL(sym_count_kernel, dim3(cdiv((size_t)n * k, T)), dim3(T), 0, s, nbr, n, k, cnt);
     RVGP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(kScanThreads), 0, s, cnt, n, start);
+    // the chunk sums of a scan sit in an array that is free then: ucnt before the
+    // sort fills it, cnt after the first scan
+    const int nb = (int)cdiv(n, kScanChunk), rows = (int)cdiv(n, kSortWaves);
+    hipLaunchKernelGGL(scan_sums_kernel, dim3(nb), dim3(kScanThreads), 0, s, cnt, n, ucnt);
     RVGP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(sym_fill_kernel, dim3(cdiv(n, T)), dim3(T), 0, s, nbr, n, k, start, cursor, tmp);
+    hipLaunchKernelGGL(scan_kernel, dim3(nb), dim3(kScanThreads), 0, s, cnt, n, ucnt, start);
     RVGP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(sym_sort_kernel, dim3(cdiv(n, T)), dim3(T), 0, s, start, n, tmp, ucnt);
+    hipLaunchKernelGGL(sym_fill_kernel, dim3(cdiv((size_t)n * k, T)), dim3(T), 0, s, nbr, n, k, start,
+                       cursor, tmp);
     RVGP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(kScanThreads), 0, s, ucnt, n, rowptr);
+    hipLaunchKernelGGL(sym_sort_kernel, dim3(rows), dim3(64 * kSortWaves), 0, s, start, n, tmp, ucnt);
     RVGP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(sym_compact_kernel, dim3(cdiv(n, T)), dim3(T), 0, s, start, n, tmp, rowptr, cols);
+    hipLaunchKernelGGL(scan_sums_kernel, dim3(nb), dim3(kScanThreads), 0, s, ucnt, n, cnt);
+    RVGP_LAUNCH_CHECK();
+    hipLaunchKernelGGL(scan_kernel, dim3(nb), dim3(kScanThreads), 0, s, ucnt, n, cnt, rowptr);
+    RVGP_LAUNCH_CHECK();
+    hipLaunchKernelGGL(sym_compact_kernel, dim3(rows), dim3(64 * kSortWaves), 0, s, start, n, tmp, rowptr,
+                       cols);
     RVGP_LAUNCH_CHECK();
     return RVGP_OK;
 }

@@ -87,10 +87,9 @@ FUSED_STEP_MAX_K = 2048  # RVGP_WS_STEP_MAX_K
 # A function-space fit of M rows works on the k x k system from M = 2 k on.
 # Its flops are ~(k / M)^3 of the M x M factorisation's; below 2 k rows
 # Phi^T Phi is singular for the tangent fields' frames (rank m d < M).
-# M = 4731, k = 200: an evaluation 10.0 -> 0.14 ms, building
-# the engine 0.84 ms.  Its
-# error against 80-bit arithmetic, noise 1 ... 1e-6, data with noise: NLML <=
-# 4e-13 and gradient <= 5e-13 (M x M: 1e-8 and 3e-8), mean 2e-13 (7e-8),
+# M = 4731, k = 200: an evaluation 10.0 -> 0.14 ms, building the engine 0.84 ms.
+# Its error against 80-bit arithmetic, noise 1 ... 1e-6, data with noise: NLML
+# <= 4e-13 and gradient <= 5e-13 (M x M: 1e-8 and 3e-8), mean 2e-13 (7e-8),
 # variance 1e-13 (5e-7); without noise, s2 -> 1e-6: gradient 1e-9 (2e-12), the
 # others as before or better.
 COEF_MIN_ROWS = 2
