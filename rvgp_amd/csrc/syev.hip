@@ -10,8 +10,7 @@
 //     its rows while forming the next reflector, so the launch boundary is
 //     the only synchronisation between workgroups (no device-scope spinning,
 //     which on gfx950 means writing back and invalidating L2 that a
-//     concurrent stream is using).  Up to kSmallN the matrix fits one
-//     workgroup's registers and one launch does all columns.
+//     concurrent stream is using).
 //  2. Eigenvalues of T by multisection (one wavefront per eigenvalue, its 64
 //     lanes evaluating Sturm counts at 64 interior points, ~9 rounds to full
 //     precision); eigenvectors of T by inverse iteration, one wavefront per
@@ -26,7 +25,7 @@
 namespace rvgp {
 
 constexpr int kSyevNB = 32;        // reflectors per compact-WY block
-constexpr int kSyevMaxN = 2048;   // inverse iteration holds 6.5 n doubles in LDS
+constexpr int kSyevMaxN = 2048;   // inverse iteration holds 5.5 n doubles in LDS
 
 // Column j of the tridiagonalisation (LAPACK sytd2, lower), one launch per
 // column on G workgroups; workgroup g owns the rows r = g (mod G) of the
@@ -322,185 +321,13 @@ __global__ __launch_bounds__(256) void copy_full_kernel(int n, const double* __r
     W[(size_t)r * ldw + c] = A[(size_t)r * lda + c];
 }
 
+__global__ void diag_one_kernel(const double* __restrict__ W, double* __restrict__ d) {
+    if (threadIdx.x == 0) d[0] = W[0];
+}
+
 __global__ void fill_kernel(size_t cnt, double* __restrict__ p, double val) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < cnt) p[i] = val;
-}
-
-// 1 / x by the hardware estimate and two Newton steps (a few units in the last
-// place): the divisions below sit on chains of n dependent steps, where the
-// IEEE sequence costs twice as much (stebz at n = 576: 369 -> 322 us).
-__device__ __forceinline__ double rcp_nr(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(fma(-x, r, 1.0), r, r);
-    return fma(fma(-x, r, 1.0), r, r);
-}
-
-// The whole tridiagonalisation of a matrix of n <= kSmallN in one workgroup,
-// the matrix in registers: wave v of NW owns the columns c = v (mod NW), lane
-// i of it the rows i + 64 k (k < R) of its C columns.  In step j every wave
-// holds the step's v, w and the next reflector u; one pass over its columns
-// applies the rank-2 update and accumulates the next product, and the one
-// column that the next reflector comes from goes through LDS (one barrier a
-// step; its two buffers alternate).  What is left is the chain of a step (the
-// barrier, NW partial products from LDS, two wave sums, the reflector's square
-// root and reciprocal), which every wave runs: a wave on each SIMD (NW = 4)
-// while its columns fit, as more waves only repeat the chain on the same SIMD
-// (16 waves: 109 us at n = 64, 4: 67 us).  A launch is 5.2 us a column, a step
-// here 1.05 us (n = 64) to 2.6 us (n = 192); the whole solve takes 516 -> 154
-// us at n = 64, 994 -> 374 us at 128, 1540 -> 729 us at 192 (200: 1600 ->
-// 1260 us, the other stages).  Past 192 the columns no longer fit the
-// registers of 8 waves.
-constexpr int kSmallN = 192;
-
-// The reflector of the column x (rows from `first` on): v with v[first] = 1
-// in place of x, and tau, beta as LAPACK's dlarfg gives them.
-template <int R>
-__device__ __forceinline__ void small_reflector(double (&x)[R], int lane, int first, double& beta,
-                                                double& tau) {
-    double alpha = 0.0, s2 = 0.0;
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const int i = lane + 64 * k;
-        if ((first >> 6) == k) alpha = bcast(x[k], first & 63);
-        x[k] = i < first ? 0.0 : x[k];
-        s2 += i == first ? 0.0 : x[k] * x[k];
-    }
-    s2 = wave_sum_dpp(s2);
-    beta = alpha;
-    tau = 0.0;
-    double scal = 0.0;
-    if (s2 != 0.0) {
-        const double nn = fma(alpha, alpha, s2);
-        double r = __builtin_amdgcn_rsq(nn);
-        r *= fma(-0.5 * nn * r, r, 1.5);
-        r *= fma(-0.5 * nn * r, r, 1.5);
-        double nrm = nn * r;
-        nrm = fma(fma(-nrm, nrm, nn), 0.5 * r, nrm);
-        beta = -copysign(nrm, alpha);
-        tau = fma(fabs(alpha), r, 1.0);
-        scal = copysign(rcp_nr(fabs(alpha) + nrm), alpha);
-    }
-#pragma unroll
-    for (int k = 0; k < R; ++k) x[k] = lane + 64 * k == first ? 1.0 : x[k] * scal;
-}
-
-template <int R>
-__device__ __forceinline__ double pick(const double (&x)[R], int i) {
-    double v = bcast(x[0], i & 63);
-#pragma unroll
-    for (int k = 1; k < R; ++k) v = (i >> 6) == k ? bcast(x[k], i & 63) : v;
-    return v;
-}
-
-template <int R, int NW>
-__global__ __launch_bounds__(64 * NW) void sytrd_small_kernel(int n, const double* __restrict__ A,
-                                                              int lda, double* __restrict__ VhT,
-                                                              double* __restrict__ d,
-                                                              double* __restrict__ e,
-                                                              double* __restrict__ tau) {
-    constexpr int C = 64 * R / NW, CG = 4;  // columns of a wave, and of one uniform skip
-    __shared__ double part[2][NW][64 * R];
-    __shared__ double next[2][64 * R];  // the column of the next reflector
-    const int lane = threadIdx.x & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    double W[C][R], u[R], p[R], nx[R];
-#pragma unroll
-    for (int q = 0; q < C; ++q) {
-        const int c = wv + NW * q;
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            const int i = lane + 64 * k;
-            W[q][k] = i < n && c < n ? A[(size_t)c * lda + i] : 0.0;
-        }
-    }
-    // the first column's reflector, its product
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const int i = lane + 64 * k;
-        u[k] = i < n ? A[i] : 0.0;
-        p[k] = 0.0;
-        if (wv == 1 % NW) next[0][i] = W[0][k];
-    }
-    double dj = bcast(u[0], 0), beta = 0.0, tj = 0.0;
-    if (n > 1) small_reflector<R>(u, lane, 1, beta, tj);
-#pragma unroll
-    for (int q = 0; q < C; ++q) {
-        const double uc = bcast(u[NW * q / 64], (wv + NW * q) & 63);  // column wv + NW q
-#pragma unroll
-        for (int k = 0; k < R; ++k) p[k] = fma(W[q][k], uc, p[k]);
-    }
-#pragma unroll
-    for (int k = 0; k < R; ++k) part[0][wv][lane + 64 * k] = p[k];
-    for (int j = 0; j + 1 < n; ++j) {
-        const int buf = j & 1;
-        if (wv == (j & (NW - 1))) {  // the outputs of step j, a wave in turn
-#pragma unroll
-            for (int k = 0; k < R; ++k) {
-                const int i = lane + 64 * k;
-                if (i > j && i < n) VhT[(size_t)j * n + i] = u[k];
-            }
-            if (lane == 0) {
-                d[j] = dj;
-                e[j] = beta;
-                tau[j] = tj;
-            }
-        }
-        __syncthreads();
-        double w[R], v[R], x[R], dot = 0.0;
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            double t = 0.0;
-#pragma unroll
-            for (int q = 0; q < NW; ++q) t += part[buf][q][lane + 64 * k];
-            v[k] = u[k];
-            w[k] = lane + 64 * k > j ? tj * t : 0.0;
-            x[k] = next[buf][lane + 64 * k];
-            dot = fma(w[k], v[k], dot);
-        }
-        const double kk = 0.5 * tj * wave_sum_dpp(dot);
-#pragma unroll
-        for (int k = 0; k < R; ++k) w[k] = fma(-kk, v[k], w[k]);
-        // column j + 1 with this step's update (v there is 1)
-        const double w1 = pick<R>(w, j + 1);
-#pragma unroll
-        for (int k = 0; k < R; ++k) u[k] = x[k] - fma(w1, v[k], w[k]);
-        dj = pick<R>(u, j + 1);
-        if (j + 2 >= n) break;
-        small_reflector<R>(u, lane, j + 2, beta, tj);
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            p[k] = 0.0;
-            nx[k] = 0.0;
-        }
-        // finished columns and those past n carry zeros in v, w or u: no test
-#pragma unroll
-        for (int g = 0; g < C; g += CG) {
-            if (NW * (g + CG) > j + 2 && NW * g < n) {
-#pragma unroll
-                for (int q = g; q < g + CG; ++q) {
-                    constexpr int S = 64 / NW;
-                    const int at = (wv + NW * q) & 63;
-                    const double vc = bcast(v[q / S], at), wc = bcast(w[q / S], at);
-                    const double uc = bcast(u[q / S], at);
-                    const bool pub = wv + NW * q == j + 2;
-#pragma unroll
-                    for (int k = 0; k < R; ++k) {
-                        W[q][k] = fma(-wc, v[k], fma(-vc, w[k], W[q][k]));
-                        p[k] = fma(W[q][k], uc, p[k]);
-                        nx[k] = pub ? W[q][k] : nx[k];
-                    }
-                }
-            }
-        }
-        const bool own = wv == ((j + 2) & (NW - 1));
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            part[buf ^ 1][wv][lane + 64 * k] = p[k];
-            if (own) next[buf ^ 1][lane + 64 * k] = nx[k];
-        }
-    }
-    if (threadIdx.x == 0) d[n - 1] = dj;
 }
 
 // Number of eigenvalues of T below x (Sturm sequence of the LDL^T pivots,
@@ -511,7 +338,7 @@ __device__ __forceinline__ int sturm_count(int n, const double* dd, const double
     if (fabs(q) <= pivmin) q = -pivmin;
     int c = q < 0.0;
     for (int i = 1; i < n; ++i) {
-        q = fma(-e2[i - 1], rcp_nr(q), dd[i] - x);
+        q = dd[i] - x - e2[i - 1] / q;
         if (fabs(q) <= pivmin) q = -pivmin;
         c += q < 0.0;
     }
@@ -592,29 +419,20 @@ __global__ __launch_bounds__(256) void tri_bounds_kernel(int n, const double* __
 // below 1e-7 |T|; its members are computed in order, each iterate
 // orthogonalised (modified Gram-Schmidt) against the members before it.
 // Eigenvector i is written to row i of Zt (n x n).  The tridiagonal
-// factorisation with partial pivoting (dlagtf) and the solves (dlagts) are
-// chains of n dependent steps: every lane walks them with the running row in
-// registers, the operands of kWalk steps are read from LDS ahead of them, and
-// the pivots' reciprocals are kept so that no solve divides.  n = 576: 650 ->
-// 247 us, n = 64: 75 -> 25 us (a cluster of four takes four times that).
-constexpr int kWalk = 8;
-
+// factorisation with partial pivoting (dlagtf) and the solve (dlagts) run on
+// lane 0; the Gram-Schmidt and normalisation use the whole wavefront.
 __global__ __launch_bounds__(64) void stein_kernel(int n, const double* __restrict__ d,
                                                    const double* __restrict__ e,
                                                    const double* __restrict__ w,
                                                    const double* __restrict__ bounds,
                                                    double* __restrict__ Zt) {
     extern __shared__ double sm[];
-    // arrays of np doubles: entries past n are the identity's, so that the
-    // walks run in whole strides
-    const int np = (n + kWalk - 1) / kWalk * kWalk + kWalk;
-    double* ra = sm;          // 1 / U diagonal
-    double* b = ra + np;      // U first super-diagonal
-    double* c = b + np;       // multipliers
-    double* dd = c + np;      // U second super-diagonal
-    double* z = dd + np;      // iterate
-    double* y = z + np;       // the iterate between the two solves; the factorisation's T
-    int* piv = reinterpret_cast<int*>(y + np);
+    double* a = sm;          // U diagonal
+    double* b = a + n;       // U first super-diagonal
+    double* c = b + n;       // multipliers
+    double* dd = c + n;      // U second super-diagonal
+    double* z = dd + n;      // iterate
+    int* piv = reinterpret_cast<int*>(z + n);
     const int lane = threadIdx.x;
     const int i0 = blockIdx.x;
     const double tn = bounds[3];
@@ -632,101 +450,62 @@ __global__ __launch_bounds__(64) void stein_kernel(int n, const double* __restri
         double lam = w[i];
         if (i > i0 && lam - lam_prev < 10.0 * eps * fabs(lam) + delta) lam = lam_prev + 10.0 * eps * fabs(lam) + delta;
         lam_prev = lam;
-        for (int k = lane; k < np; k += 64) {
-            y[k] = k < n ? d[k] - lam : 1.0;      // diagonal
-            z[k] = k < n - 1 ? e[k] : 0.0;        // off-diagonal
-        }
-        __syncthreads();
-        double ak = y[0], bk = z[0];  // row k of U in the making
-        for (int k0 = 0; k0 < n; k0 += kWalk) {
-            double de[kWalk], ee[kWalk + 1];
-#pragma unroll
-            for (int q = 0; q < kWalk; ++q) {
-                de[q] = y[k0 + q + 1];
-                ee[q] = z[k0 + q];
+        if (lane == 0) {
+            for (int k = 0; k < n; ++k) {
+                a[k] = d[k] - lam;
+                b[k] = k < n - 1 ? e[k] : 0.0;
+                c[k] = k < n - 1 ? e[k] : 0.0;
+                dd[k] = 0.0;
+                piv[k] = 0;
             }
-            ee[kWalk] = z[k0 + kWalk];
-            double r[kWalk], bo[kWalk], mo[kWalk], so[kWalk];
-            int po[kWalk];
-#pragma unroll
-            for (int q = 0; q < kWalk; ++q) {
-                const double ck = ee[q], dn = de[q], en = ee[q + 1];
-                const bool swap = fmax(fabs(ak), delta) < fabs(ck);
-                const double floored = fabs(ak) < delta ? copysign(delta, ak == 0.0 ? 1.0 : ak) : ak;
-                r[q] = rcp_nr(swap ? ck : floored);
-                const double mult = (swap ? ak : ck) * r[q];
-                bo[q] = swap ? dn : bk;
-                so[q] = swap ? en : 0.0;
-                mo[q] = mult;
-                po[q] = swap;
-                const double na = fma(-mult, swap ? dn : bk, swap ? bk : dn);
-                bk = swap ? -mult * en : en;
-                ak = na;
-            }
-            if (lane == 0) {
-#pragma unroll
-                for (int q = 0; q < kWalk; ++q) {
-                    ra[k0 + q] = r[q];
-                    b[k0 + q] = bo[q];
-                    c[k0 + q] = mo[q];
-                    dd[k0 + q] = so[q];
-                    piv[k0 + q] = po[q];
+            for (int k = 0; k < n - 1; ++k) {
+                if (fabs(a[k]) >= fabs(c[k])) {
+                    const double ak = fabs(a[k]) < delta ? copysign(delta, a[k] == 0.0 ? 1.0 : a[k]) : a[k];
+                    a[k] = ak;
+                    const double mult = c[k] / ak;
+                    c[k] = mult;
+                    a[k + 1] -= mult * b[k];
+                    dd[k] = 0.0;
+                    piv[k] = 0;
+                } else {
+                    const double mult = a[k] / c[k];
+                    a[k] = c[k];
+                    const double temp = a[k + 1];
+                    a[k + 1] = b[k] - mult * temp;
+                    if (k < n - 2) {
+                        dd[k] = b[k + 1];
+                        b[k + 1] = -mult * dd[k];
+                    }
+                    b[k] = temp;
+                    c[k] = mult;
+                    piv[k] = 1;
                 }
             }
+            if (fabs(a[n - 1]) < delta) a[n - 1] = copysign(delta, a[n - 1] == 0.0 ? 1.0 : a[n - 1]);
         }
-        __syncthreads();
         // deterministic, non-degenerate starting vector
-        for (int k = lane; k < np; k += 64) {
+        for (int k = lane; k < n; k += 64) {
             const unsigned h = (unsigned)(k * 2654435761u) ^ (unsigned)(i * 40503u + 17u);
-            z[k] = k < n ? 0.5 + (double)(h & 0xffff) / 65536.0 : 0.0;
+            z[k] = 0.5 + (double)(h & 0xffff) / 65536.0;
         }
         __syncthreads();
         for (int it = 0; it < 3; ++it) {
-            // forward: the row interchanges and multipliers, z -> y
-            double zk = z[0];
-            for (int k0 = 0; k0 < n; k0 += kWalk) {
-                double zn[kWalk], ck[kWalk];
-                int pk[kWalk];
-#pragma unroll
-                for (int q = 0; q < kWalk; ++q) {
-                    zn[q] = z[k0 + q + 1];
-                    ck[q] = c[k0 + q];
-                    pk[q] = piv[k0 + q];
+            if (lane == 0) {
+                // forward: apply the row interchanges and multipliers
+                for (int k = 0; k < n - 1; ++k) {
+                    if (piv[k] == 0) {
+                        z[k + 1] -= c[k] * z[k];
+                    } else {
+                        const double tmp = z[k];
+                        z[k] = z[k + 1];
+                        z[k + 1] = tmp - c[k] * z[k];
+                    }
                 }
-#pragma unroll
-                for (int q = 0; q < kWalk; ++q) {
-                    const double keep = pk[q] ? zn[q] : zk, go = pk[q] ? zk : zn[q];
-                    zn[q] = keep;
-                    zk = fma(-ck[q], keep, go);
-                }
-                if (lane == 0) {
-#pragma unroll
-                    for (int q = 0; q < kWalk; ++q) y[k0 + q] = zn[q];
-                }
-            }
-            __syncthreads();
-            // back substitution with U, y -> z
-            double z1 = 0.0, z2 = 0.0;
-            for (int k0 = (n + kWalk - 1) / kWalk * kWalk - kWalk; k0 >= 0; k0 -= kWalk) {
-                double yk[kWalk], bq[kWalk], dq[kWalk], rq[kWalk];
-#pragma unroll
-                for (int q = 0; q < kWalk; ++q) {
-                    yk[q] = y[k0 + q];
-                    bq[q] = b[k0 + q];
-                    dq[q] = dd[k0 + q];
-                    rq[q] = ra[k0 + q];
-                }
-#pragma unroll
-                for (int q = kWalk - 1; q >= 0; --q) {
-                    const double v = k0 + q < n ? fma(-bq[q], z1, fma(-dq[q], z2, yk[q])) * rq[q] : 0.0;
-                    z2 = z1;
-                    z1 = v;
-                    yk[q] = v;
-                }
-                if (lane == 0) {
-#pragma unroll
-                    for (int q = 0; q < kWalk; ++q) z[k0 + q] = yk[q];
-                }
+                // back substitution with U (diag a, supers b, dd)
+                z[n - 1] /= a[n - 1];
+                if (n > 1) z[n - 2] = (z[n - 2] - b[n - 2] * z[n - 1]) / a[n - 2];
+                for (int k = n - 3; k >= 0; --k)
+                    z[k] = (z[k] - b[k] * z[k + 1] - dd[k] * z[k + 2]) / a[k];
             }
             __syncthreads();
             // orthogonalise against the cluster's earlier members, normalise
@@ -734,7 +513,7 @@ __global__ __launch_bounds__(64) void stein_kernel(int n, const double* __restri
                 const double* zq = Zt + (size_t)q * n;
                 double s = 0.0;
                 for (int k = lane; k < n; k += 64) s += zq[k] * z[k];
-                s = wave_sum_dpp(s);
+                s = wave_sum(s);
                 for (int k = lane; k < n; k += 64) z[k] -= s * zq[k];
                 __syncthreads();
             }
@@ -749,7 +528,7 @@ __global__ __launch_bounds__(64) void stein_kernel(int n, const double* __restri
                 const double zk = z[k] * sc;
                 nrm += zk * zk;
             }
-            nrm = wave_sum_dpp(nrm);
+            nrm = wave_sum(nrm);
             const double inv = nrm > 0.0 ? sc / sqrt(nrm) : 1.0;
             __syncthreads();
             for (int k = lane; k < n; k += 64) z[k] *= inv;
@@ -771,214 +550,175 @@ __global__ __launch_bounds__(64) void stein_kernel(int n, const double* __restri
     }
 }
 
-using dbl4 = double __attribute__((ext_vector_type(4)));
-
-// Block reflectors (LAPACK larft, forward, columnwise): Vb (I - Vb Tb Vb^T =
-// H_j0 ... H_{j0+NB-1}, Vb = VhT[j0:j0+NB]^T) as VT = Vb Tb, row q of the block
-// in VT[j0 + q].  One workgroup per block.  The Gram G = Vb^T Vb and Vb Tb are
-// on the matrix cores; row p of Tb depends on itself and G only, so lane p
-// holds it in registers and the recursion needs no barrier.  n = 64: 41 ->
-// 9 us, n = 576: 87 -> 22 us.
-constexpr int kLarftWaves = 8;
-
-__global__ __launch_bounds__(64 * kLarftWaves) void larft_kernel(int n, int nref,
-                                                                 const double* __restrict__ VhT,
-                                                                 const double* __restrict__ tau,
-                                                                 double* __restrict__ VT) {
-    constexpr int NB = kSyevNB, LD = NB + 1;
-    __shared__ double G[kLarftWaves][NB * LD];  // partial Grams, their sum in G[0]; Tb in G[1]
-    const int lane = threadIdx.x & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m = lane & 15, kq = lane >> 4;
-    const int j0 = blockIdx.x * NB;
-    const double* V0 = VhT + (size_t)(j0 + m) * n;
-    const double* V1 = V0 + (size_t)16 * n;
-    const bool ok0 = j0 + m < nref, ok1 = j0 + 16 + m < nref;
-    dbl4 g00 = dbl4{0, 0, 0, 0}, g01 = g00, g11 = g00;
-    for (int r0 = j0 + 16 * wv; r0 < n; r0 += 16 * kLarftWaves) {
-        double a0[4], a1[4];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int r = r0 + 4 * kq + s;
-            a0[s] = ok0 && r < n ? V0[r] : 0.0;
-            a1[s] = ok1 && r < n ? V1[r] : 0.0;
+// Triangular factor of each block of NB reflectors (LAPACK larft, forward,
+// columnwise): I - Vb Tb Vb^T = H_j0 ... H_{j0+nb-1}, Vb = VhT[j0:j0+nb]^T.
+// One workgroup per block; the Gram G = Vb^T Vb one wavefront per entry.
+__global__ __launch_bounds__(256) void larft_kernel(int n, int nref, const double* __restrict__ VhT,
+                                                    const double* __restrict__ tau,
+                                                    double* __restrict__ Tb) {
+    constexpr int NB = kSyevNB;
+    __shared__ double G[NB][NB + 1], T[NB][NB + 1];
+    const int blk = blockIdx.x;
+    const int j0 = blk * NB;
+    const int nb = min(NB, nref - j0);
+    __shared__ double Vs[NB][129];
+    for (int e = threadIdx.x; e < NB * (NB + 1); e += 256) {
+        (&G[0][0])[e] = 0.0;
+        (&T[0][0])[e] = 0.0;
+    }
+    // G = Vb^T Vb over row chunks of 128 staged in LDS; thread -> entries
+    // (p, q) with p <= q, at most 3 per thread (528 for NB = 32)
+    double gacc[3] = {0.0, 0.0, 0.0};
+    for (int r0 = j0 + 1; r0 < n; r0 += 128) {
+        __syncthreads();
+        for (int e = threadIdx.x; e < NB * 128; e += 256) {
+            const int p = e >> 7, c = e & 127;
+            const int r = r0 + c;
+            Vs[p][c] = (p < nb && r < n) ? VhT[(size_t)(j0 + p) * n + r] : 0.0;
         }
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            g00 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[s], a0[s], g00, 0, 0, 0);
-            g01 = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[s], a1[s], g01, 0, 0, 0);
-            g11 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[s], a1[s], g11, 0, 0, 0);
+        __syncthreads();
+        for (int k = 0; k < 3; ++k) {
+            const int idx = threadIdx.x + 256 * k;
+            if (idx >= NB * (NB + 1) / 2) break;
+            int p = 0, rem = idx;
+            while (rem >= NB - p) { rem -= NB - p; ++p; }
+            const int q = p + rem;
+            double sacc = 0.0;
+            for (int c = 0; c < 128; ++c) sacc += Vs[p][c] * Vs[q][c];
+            gacc[k] += sacc;
         }
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {  // element r of a lane: row lane/16 + 4 r, column lane%16
-        const int row = kq + 4 * r;
-        G[wv][row * LD + m] = g00[r];
-        G[wv][row * LD + 16 + m] = g01[r];
-        G[wv][(16 + row) * LD + 16 + m] = g11[r];
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < NB * NB; i += 64 * kLarftWaves) {
-        const int at = (i / NB) * LD + i % NB;
-        if (i % NB > i / NB) {
-            double v = 0.0;
-#pragma unroll
-            for (int q = 0; q < kLarftWaves; ++q) v += G[q][at];
-            G[0][at] = v;
-        }
+    for (int k = 0; k < 3; ++k) {
+        const int idx = threadIdx.x + 256 * k;
+        if (idx >= NB * (NB + 1) / 2) break;
+        int p = 0, rem = idx;
+        while (rem >= NB - p) { rem -= NB - p; ++p; }
+        G[p][p + rem] = gacc[k];
     }
     __syncthreads();
-    if (wv == 0) {
-        const int p = lane & (NB - 1);
-        const double tp = j0 + p < nref ? tau[j0 + p] : 0.0;
-        double T[NB];
-        int col = 0;
-#pragma unroll
-        for (int q = 0; q < NB; ++q) {  // T[p][q] = -tau_q sum_{l<q} T[p][l] G[l][q]
-            double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-            for (int l = 0; l + 1 < q; l += 2) {
-                s0 = fma(T[l], G[0][l * LD + col], s0);
-                s1 = fma(T[l + 1], G[0][(l + 1) * LD + col], s1);
-            }
-            if (q & 1) s0 = fma(T[q - 1], G[0][(q - 1) * LD + col], s0);
-            const double tq = bcast(tp, q);
-            T[q] = q == p ? tq : q > p ? -tq * (s0 + s1) : 0.0;
-            // the next column's address waits for this one: all 496 reads
-            // hoisted would spill
-            ++col;
-            asm volatile("" : "+v"(col), "+v"(T[q]));
+    for (int q = 0; q < nb; ++q) {
+        // T[0:q, q] = -tau_q T[0:q, 0:q] G[0:q, q]
+        const double tq = tau[j0 + q];
+        if ((int)threadIdx.x < q) {
+            const int p = threadIdx.x;
+            double sacc = 0.0;
+            for (int l = p; l < q; ++l) sacc += T[p][l] * G[l][q];
+            T[p][q] = -tq * sacc;
         }
-        // one wave, LDS in order: no lane still reads G here
-        if (lane < NB) {
-#pragma unroll
-            for (int q = 0; q < NB; ++q) G[1][p * LD + q] = T[q];
-        }
+        if (threadIdx.x == 0) T[q][q] = tq;
+        __syncthreads();
     }
-    __syncthreads();
-    // VT^T = Tb^T Vb^T
-    double at[2][8];
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        at[0][s] = G[1][(4 * s + kq) * LD + m];
-        at[1][s] = G[1][(4 * s + kq) * LD + 16 + m];
-    }
-    for (int r0 = j0 + 16 * wv; r0 < n; r0 += 16 * kLarftWaves) {
-        const int r = r0 + m;
-        double b[8];
-#pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            const int p = j0 + 4 * s + kq;
-            b[s] = p < nref && r < n ? VhT[(size_t)p * n + r] : 0.0;
-        }
-        dbl4 acc0 = dbl4{0, 0, 0, 0}, acc1 = acc0;
-#pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(at[0][s], b[s], acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(at[1][s], b[s], acc1, 0, 0, 0);
-        }
-        if (r < n) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int q = j0 + kq + 4 * e;
-                if (q < nref) VT[(size_t)q * n + r] = acc0[e];
-                if (q + 16 < nref) VT[(size_t)(q + 16) * n + r] = acc1[e];
-            }
-        }
+    for (int e = threadIdx.x; e < NB * NB; e += 256) {
+        const int p = e / NB, q = e - p * NB;
+        Tb[(size_t)blk * NB * NB + e] = (p < nb && q < nb) ? T[p][q] : 0.0;
     }
 }
 
 // V = H_0 H_1 ... H_{n-2} Z, Z = Zt^T (Zt row i = eigenvector i of T).
 // Columns are independent under a left product, so workgroup c0 takes NC
-// columns of Z into LDS and applies the reflector blocks last to first:
-// Y = Vb^T Z (the rows split over four groups of two waves, a 16-row half of Y
-// each), then Z -= (Vb Tb) Y by 16-row tiles, both on the matrix cores with
-// the reflectors read from L2.  Two barriers a block.  NC = 16 fills a matrix
-// instruction; 8 where 16 columns of Z pass LDS.  n = 64: 26 -> 7 us,
-// n = 576: 700 -> 147 us, n = 1000: 2070 -> 360 us.
-constexpr int kApplyWaves = 8;
-
+// columns of Z into LDS and applies the reflector blocks last to first in
+// compact WY form: Y1 = Vb^T Z, Y2 = Tb Y1, Z -= Vb Y2, streaming each
+// block's reflectors (rows j0.. of VhT) through LDS in chunks of 128 rows.
 template <int NC>
-__global__ __launch_bounds__(64 * kApplyWaves) void apply_q_kernel(int n, int nref,
-                                                                   const double* __restrict__ VhT,
-                                                                   const double* __restrict__ VT,
-                                                                   const double* __restrict__ Zt,
-                                                                   double* __restrict__ V, int ldv) {
-    constexpr int NB = kSyevNB, KS = kApplyWaves / 2;
+__global__ __launch_bounds__(256) void apply_q_kernel(int n, int nref, const double* __restrict__ VhT,
+                                                      const double* __restrict__ Tb,
+                                                      const double* __restrict__ Zt,
+                                                      double* __restrict__ V, int ldv) {
+    constexpr int NB = kSyevNB, RC = 128;
     extern __shared__ double sm[];
-    const int n16 = (n + 15) & ~15;
-    double* Z = sm;                          // n16 x NC, zero past n
-    double* Y = Z + (size_t)n16 * NC;        // KS partial Y, NB x NC each
-    const int t = threadIdx.x, lane = t & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int m = lane & 15, kq = lane >> 4;
-    const bool cok = m < NC;
+    double* Z = sm;                                // n x NC
+    double* Vs = Z + (size_t)n * NC;               // NB x (RC + 1)
+    double* Y = Vs + NB * (RC + 1);                // NB x NC
+    double* Ts = Y + NB * NC;                      // NB x (NB + 1)
+    const int t = threadIdx.x;
     const int c0 = blockIdx.x * NC;
-    for (int e = t; e < n16 * NC; e += 64 * kApplyWaves) {
-        const int c = e / n16, r = e - c * n16;  // coalesced over r
-        Z[r * NC + c] = c0 + c < n && r < n ? Zt[(size_t)(c0 + c) * n + r] : 0.0;
+    const int ncol = min(NC, n - c0);
+    for (int e = t; e < n * NC; e += 256) {
+        const int c = e / n, r = e - c * n;         // coalesced over r
+        Z[r * NC + c] = c < ncol ? Zt[(size_t)(c0 + c) * n + r] : 0.0;
     }
     const int nblk = (nref + NB - 1) / NB;
     for (int b = nblk - 1; b >= 0; --b) {
         const int j0 = b * NB;
+        const int nb = min(NB, nref - j0);
         __syncthreads();
-        {
-            const int p = j0 + 16 * (wv & 1) + m, g = wv >> 1;
-            const double* Vp = VhT + (size_t)p * n;
-            dbl4 acc = dbl4{0, 0, 0, 0};
-            for (int r0 = j0 + 16 * g; r0 < n; r0 += 16 * KS) {
-                double a[4], z[4];
+        for (int e = t; e < NB * NB; e += 256) Ts[(e / NB) * (NB + 1) + e % NB] = Tb[(size_t)b * NB * NB + e];
+        // Y1 = Vb^T Z: thread -> (p, c) entries
+        double y1[(NB * NC + 255) / 256];
 #pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const int r = r0 + 4 * kq + s;
-                    a[s] = p < nref && r < n ? Vp[r] : 0.0;
-                    z[s] = cok ? Z[r * NC + m] : 0.0;
+        for (int k = 0; k < (NB * NC + 255) / 256; ++k) y1[k] = 0.0;
+        for (int r0 = j0 + 1; r0 < n; r0 += RC) {
+            __syncthreads();
+            for (int e = t; e < NB * RC; e += 256) {
+                const int p = e / RC, cc = e - p * RC;
+                const int r = r0 + cc;
+                Vs[p * (RC + 1) + cc] = (p < nb && r < n) ? VhT[(size_t)(j0 + p) * n + r] : 0.0;
+            }
+            __syncthreads();
+            const int rl = min(RC, n - r0);
+#pragma unroll
+            for (int k = 0; k < (NB * NC + 255) / 256; ++k) {
+                const int idx = t + 256 * k;
+                if (idx < NB * NC) {
+                    const int p = idx / NC, c = idx - p * NC;
+                    double sacc = 0.0;
+                    for (int cc = 0; cc < rl; ++cc) sacc += Vs[p * (RC + 1) + cc] * Z[(r0 + cc) * NC + c];
+                    y1[k] += sacc;
                 }
-#pragma unroll
-                for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], z[s], acc, 0, 0, 0);
-            }
-            if (cok) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) Y[(g * NB + 16 * (wv & 1) + kq + 4 * r) * NC + m] = acc[r];
             }
         }
         __syncthreads();
-        double y[8];
+        // Y2 = Tb Y1 (Tb upper triangular)
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            double v = 0.0;
-#pragma unroll
-            for (int g = 0; g < KS; ++g) v += cok ? Y[(g * NB + 4 * s + kq) * NC + m] : 0.0;
-            y[s] = -v;
+        for (int k = 0; k < (NB * NC + 255) / 256; ++k) {
+            const int idx = t + 256 * k;
+            if (idx < NB * NC) Y[idx] = y1[k];
         }
-        for (int r0 = j0 + 16 * wv; r0 < n; r0 += 16 * kApplyWaves) {
-            const int r = r0 + m;
-            double a[8];
+        __syncthreads();
+        double y2[(NB * NC + 255) / 256];
 #pragma unroll
-            for (int s = 0; s < 8; ++s) {
-                const int p = j0 + 4 * s + kq;
-                a[s] = p < nref && r < n ? VT[(size_t)p * n + r] : 0.0;
+        for (int k = 0; k < (NB * NC + 255) / 256; ++k) {
+            const int idx = t + 256 * k;
+            y2[k] = 0.0;
+            if (idx < NB * NC) {
+                const int p = idx / NC, c = idx - p * NC;
+                for (int l = p; l < NB; ++l) y2[k] += Ts[p * (NB + 1) + l] * Y[l * NC + c];
             }
-            dbl4 acc;
+        }
+        __syncthreads();
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] = cok ? Z[(r0 + kq + 4 * e) * NC + m] : 0.0;
-#pragma unroll
-            for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], y[s], acc, 0, 0, 0);
-            if (cok) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) Z[(r0 + kq + 4 * e) * NC + m] = acc[e];
+        for (int k = 0; k < (NB * NC + 255) / 256; ++k) {
+            const int idx = t + 256 * k;
+            if (idx < NB * NC) Y[idx] = y2[k];
+        }
+        // Z -= Vb Y2, chunk by chunk
+        for (int r0 = j0 + 1; r0 < n; r0 += RC) {
+            __syncthreads();
+            for (int e = t; e < NB * RC; e += 256) {
+                const int p = e / RC, cc = e - p * RC;
+                const int r = r0 + cc;
+                Vs[p * (RC + 1) + cc] = (p < nb && r < n) ? VhT[(size_t)(j0 + p) * n + r] : 0.0;
+            }
+            __syncthreads();
+            const int rl = min(RC, n - r0);
+            for (int e = t; e < rl * NC; e += 256) {
+                const int cc = e / NC, c = e - cc * NC;
+                double sacc = 0.0;
+#pragma unroll 8
+                for (int p = 0; p < NB; ++p) sacc += Vs[p * (RC + 1) + cc] * Y[p * NC + c];
+                Z[(r0 + cc) * NC + c] -= sacc;
             }
         }
     }
     __syncthreads();
-    for (int e = t; e < n * NC; e += 64 * kApplyWaves) {
+    for (int e = t; e < n * NC; e += 256) {
         const int r = e / NC, c = e - r * NC;
-        if (c0 + c < n) V[(size_t)r * ldv + c0 + c] = Z[e];
+        if (c < ncol) V[(size_t)r * ldv + c0 + c] = Z[e];
     }
 }
 
 struct SyevWs {
-    size_t d, e, tau, bounds, W, Vh, vb, pb, sb, Zt, total;
+    size_t d, e, tau, bounds, W, Vh, vb, pb, sb, Zt, Tb, total;
     int ldw;
 };
 
@@ -990,6 +730,7 @@ static SyevWs syev_layout(int n) {
         off += align_up(doubles * sizeof(double), 256);
         return o;
     };
+    const int nblk = (n + kSyevNB - 1) / kSyevNB;
     L.d = take(n);
     L.e = take(n);
     L.tau = take(n);
@@ -1001,6 +742,7 @@ static SyevWs syev_layout(int n) {
     L.pb = take(2 * (size_t)n);
     L.sb = take(2 * (size_t)kStepGroupsMax);
     L.Zt = take((size_t)n * n);
+    L.Tb = take((size_t)nblk * kSyevNB * kSyevNB);
     L.total = off;
     return L;
 }
@@ -1033,26 +775,22 @@ extern "C" int rvgp_syev(int n, double* A, int lda, double* w, double* V, int ld
     double* Wp = reinterpret_cast<double*>(base + L.pb);
     double* sb = reinterpret_cast<double*>(base + L.sb);
     double* Zt = reinterpret_cast<double*>(base + L.Zt);
+    double* Tb = reinterpret_cast<double*>(base + L.Tb);
     const int ldw = L.ldw;
 
     // stage 1: tridiagonalisation, one launch per column (reflectors
     // j = 0 .. n-2; the last has length 1 and tau = 0)
     const size_t nn = (size_t)n * n;
-    if (n > kSmallN) {
-        hipLaunchKernelGGL(copy_full_kernel, dim3(cdiv(nn, 256)), dim3(256), 0, s, n, A, lda, W, ldw);
-        RVGP_LAUNCH_CHECK();
-    }
+    hipLaunchKernelGGL(copy_full_kernel, dim3(cdiv(nn, 256)), dim3(256), 0, s, n, A, lda, W, ldw);
+    RVGP_LAUNCH_CHECK();
     hipLaunchKernelGGL(fill_kernel, dim3(cdiv(nn, 256)), dim3(256), 0, s, nn, VhT, 0.0);
     RVGP_LAUNCH_CHECK();
-    const size_t stsm = sizeof(double) * (4 * (size_t)n + 2 * (kStepThreads / 64));
-    if (n <= kSmallN) {
-        const int rows = cdiv(n, 64);
-        const auto kern = rows == 1   ? sytrd_small_kernel<1, 4>
-                          : rows == 2 ? sytrd_small_kernel<2, 4>
-                                      : sytrd_small_kernel<3, 8>;
-        hipLaunchKernelGGL(kern, dim3(1), dim3(rows < 3 ? 256 : 512), 0, s, n, A, lda, VhT, d, e, tau);
+    if (n == 1) {
+        hipLaunchKernelGGL(diag_one_kernel, dim3(1), dim3(64), 0, s, W, d);
         RVGP_LAUNCH_CHECK();
-    } else if (n <= 1024) {
+    }
+    const size_t stsm = sizeof(double) * (4 * (size_t)n + 2 * (kStepThreads / 64));
+    if (n <= 1024) {
         // 128 workgroups x 4 wavefronts x 2 rows cover the <= 1023 trailing rows
         const int G = n < kStepGroupsMax ? n : kStepGroupsMax;
         auto kern = sytrd_step_prefetch_kernel<2, 16>;
@@ -1080,8 +818,7 @@ extern "C" int rvgp_syev(int n, double* A, int lda, double* w, double* V, int ld
     hipLaunchKernelGGL(stebz_kernel, dim3(n), dim3(64), sizeof(double) * 2 * n, s, n, d, e, bounds,
                        w);
     RVGP_LAUNCH_CHECK();
-    const size_t np = (n + kWalk - 1) / kWalk * kWalk + kWalk;
-    const size_t ssm = (sizeof(double) * 6 + sizeof(int)) * np;
+    const size_t ssm = sizeof(double) * 5 * n + sizeof(int) * n;
     RVGP_CHECK_HIP(hipFuncSetAttribute((const void*)stein_kernel,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)ssm));
     hipLaunchKernelGGL(stein_kernel, dim3(n), dim3(64), ssm, s, n, d, e, w, bounds, Zt);
@@ -1089,17 +826,24 @@ extern "C" int rvgp_syev(int n, double* A, int lda, double* w, double* V, int ld
     // stage 3: V = H_0 H_1 ... H_{n-2} Z with Z = Zt^T (one fused kernel,
     // a few columns of Z per workgroup)
     const int nblk = (nref + kSyevNB - 1) / kSyevNB;
-    if (nblk > 0) {  // W is free by now: it takes Vb Tb
-        hipLaunchKernelGGL(larft_kernel, dim3(nblk), dim3(64 * kLarftWaves), 0, s, n, nref, VhT, tau, W);
+    if (nblk > 0) {
+        hipLaunchKernelGGL(larft_kernel, dim3(nblk), dim3(256), 0, s, n, nref, VhT, tau, Tb);
         RVGP_LAUNCH_CHECK();
     }
-    const int nc = n <= 1024 ? 16 : 8;
-    const size_t qsm = sizeof(double) * nc * ((size_t)((n + 15) & ~15) + (kApplyWaves / 2) * kSyevNB);
-    const auto apply = nc == 16 ? apply_q_kernel<16> : apply_q_kernel<8>;
-    RVGP_CHECK_HIP(hipFuncSetAttribute((const void*)apply, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)qsm));
-    hipLaunchKernelGGL(apply, dim3(cdiv(n, nc)), dim3(64 * kApplyWaves), qsm, s, n, nref, VhT, W, Zt, V,
-                       ldv);
+    const int nc = n <= 1024 ? 8 : 4;
+    const size_t qsm = sizeof(double) * ((size_t)n * nc + kSyevNB * 129 + kSyevNB * nc +
+                                         kSyevNB * (kSyevNB + 1));
+    if (nc == 8) {
+        RVGP_CHECK_HIP(hipFuncSetAttribute((const void*)apply_q_kernel<8>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)qsm));
+        hipLaunchKernelGGL(apply_q_kernel<8>, dim3(cdiv(n, 8)), dim3(256), qsm, s, n, nref, VhT, Tb,
+                           Zt, V, ldv);
+    } else {
+        RVGP_CHECK_HIP(hipFuncSetAttribute((const void*)apply_q_kernel<4>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)qsm));
+        hipLaunchKernelGGL(apply_q_kernel<4>, dim3(cdiv(n, 4)), dim3(256), qsm, s, n, nref, VhT, Tb,
+                           Zt, V, ldv);
+    }
     RVGP_LAUNCH_CHECK();
     return RVGP_OK;
 }
