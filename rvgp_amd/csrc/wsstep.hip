@@ -287,7 +287,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 // one cubic step), a product and an update; rows and columns are scaled at the
 // end, each lane taking its pivot's inverse square root.  Entries of other
 // lanes come by DPP broadcasts (v_readlane and the hazard of its scalar result
-// took twice as long).  A step at k = 500: 223 -> 190 us.
+// took twice as long).  A step at k = 500: 215 -> 183 us.
 __device__ __forceinline__ void chol_inv16(const double* C, int ldc, double* L, double* D, int ldo,
                                            int lane, int& bad) {
     const int i = lane & 15;
