@@ -437,16 +437,16 @@ int rvgp_ws_step(int k, int typ, const double* evals, double n_rows, const doubl
                  double b1, double b2, double eps, void* ws, size_t ws_bytes, int* sync,
                  size_t sync_ints, double* out, int* status, void* stream);
 
-/* rvgp_ws_step from the least-squares split of the observations, y = Phi c + e
- * with Phi^T e = 0: c (k) beside b, ee = |e|^2 in place of yy.  The same
- * NLML, gradient and update, with no cancellation at small noise (the
- * function-space form's accuracy at the weight-space form's cost).  Workspace,
- * sync and status as rvgp_ws_step. */
+/* rvgp_ws_step from a split of the observations, y = Phi c + e: c (k) and
+ * ge = Phi^T e (k) beside b, ee = |e|^2 in place of yy.  Any c serves; near the
+ * least-squares one, where ge is small, nothing cancels at small noise (the
+ * function-space form's accuracy at the weight-space form's cost).  The same
+ * NLML, gradient and update; workspace, sync and status as rvgp_ws_step. */
 int rvgp_coef_step(int k, int typ, const double* evals, double n_rows, const double* G, int ldg,
-                   const double* b, const double* c, const double* ee, double M,
-                   const double* lower, double* u, const int* trainable, double* m1, double* m2, double* t, int do_adam, double lr,
-                   double b1, double b2, double eps, void* ws, size_t ws_bytes, int* sync,
-                   size_t sync_ints, double* out, int* status, void* stream);
+                   const double* b, const double* c, const double* ge, const double* ee, double M,
+                   const double* lower, double* u, const int* trainable, double* m1, double* m2,
+                   double* t, int do_adam, double lr, double b1, double b2, double eps, void* ws,
+                   size_t ws_bytes, int* sync, size_t sync_ints, double* out, int* status, void* stream);
 
 /* ---------------------------------------------------------------------
  * Batched fits: F independent fields on one manifold, each with its own

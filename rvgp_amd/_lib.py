@@ -82,7 +82,7 @@ SIGNATURES = {
     "rvgp_ws_step_sync_ints": (S, [I]),
     "rvgp_ws_step": (I, [I, I, P, D, P, I, P, P, D, P, P, P, P, P, P, I, D, D, D, D, P, S, P, S,
                          P, P, P]),
-    "rvgp_coef_step": (I, [I, I, P, D, P, I, P, P, P, D, P, P, P, P, P, P, I, D, D, D, D, P, S, P, S,
+    "rvgp_coef_step": (I, [I, I, P, D, P, I, P, P, P, P, D, P, P, P, P, P, P, I, D, D, D, D, P, S, P, S,
                            P, P, P]),
     "rvgp_batch_gram": (I, [I, I, I, I, P, I, P, P, I, P, P]),
     "rvgp_batch_rhs": (I, [I, I, I, P, I, P, P, P, P, P, P, P]),

@@ -21,11 +21,22 @@
 //           squares of X(i,j), i >= j                        (w = X^T X b),
 //           and tile j's share of every sum the NLML and adjoint need
 //   final   NLML, adjoint, Adam; advances the epoch.
+// With `refine`, where the pivots of a diagonal tile have lost most of A's diagonal
+// (kIll), the tiles below it are corrected by their residual C - L(i,j) L(j,j)^T;
+// where any tile's have, the columns only give w, and three more sets of tasks
+// take one step of iterative refinement before the sums are formed:
+//   residual i  r_i = b_i - s2 w_i / S_i - (G w)_i
+//   row' i      t_i = sum_{j<=i} X(i,j) r_j
+//   col' j      w_j += sum_{i>=j} X(i,j)^T t_i, and the sums
+// Explicit inverses of tiles leave an error of cond(L) that solves with L do
+// not: with nodes on a part of the manifold (M = 500, k = 130, G singular to
+// working precision, s2 = 1e-4 and 2e-6) the NLML was off by 2e-4 and 0.6
+// without all this, by 8e-8 and 2e-5 with it.
 // Tasks are numbered (L tasks column by column, then X tasks column by
-// column, filter, rows, columns, final) so that every task depends only on tasks
-// with smaller block indices: the dispatcher starts workgroups in index
-// order, so a waiting workgroup never holds a slot its producer needs, and
-// the grid drains for any number of resident workgroups.
+// column, filter, rows, columns, refinement, final) so that every task depends
+// only on tasks with smaller block indices: the dispatcher starts workgroups in
+// index order, so a waiting workgroup never holds a slot its producer needs,
+// and the grid drains for any number of resident workgroups.
 //
 // Synchronisation (HIP/HSA memory model, agent scope): a producer's every
 // wave waits until its stores have reached the L2, the workgroup meets at a
@@ -33,7 +44,9 @@
 // written back) and stores the flag; a consumer's lane 0 polls the flag with relaxed agent-scope
 // loads, issues an agent-scope acquire fence (L1/L2 invalidation) and the
 // workgroup meets at a barrier before reading.  Flags hold the step's epoch
-// (sync[ctl]), so nothing is cleared between steps.  Every wait is bounded:
+// (sync[ctl]), so nothing is cleared between steps; the refinement raises the
+// rows' flags to epoch + 1 (residual) and + 2 (row'), the columns' to epoch + 1,
+// and the step then ends at epoch + 2.  Every wait is bounded:
 // past kSpinLimit polls -- or once another workgroup has given up -- it sets
 // an error flag and continues, the step completes with garbage and status
 // RVGP_ST_TIMEOUT; no launch can hang.
@@ -56,6 +69,12 @@ constexpr int kSpinLimit = 1 << 21;
 // Filter values that an optimiser's trial step sends to 0 (a sigma_f of 1e-300,
 // a steep filter): 1 / S stays finite, S itself is as good as 0.
 constexpr double kMinS = 1e-280;
+// L_qq^2 / A_qq below which explicit inverses lose more than a digit.  (At 1e-4
+// the NLML of 300 rows on half a circle, s2 = 1e-4, was off by 3e-5 unnoticed.)
+// Rows of nodes all over the manifold stay far above: such a step takes as long
+// as without the test (88 us at k = 200, 185 us at 500), a refined one 111 and
+// 229 us.
+constexpr double kIll = 1e-2;
 
 // task numbering.  L column j: the diagonal task (which also produces
 // L(j+1,j)), then L(i,j) for i >= j+2; X column j: X(i,j) for i > j.
@@ -68,7 +87,7 @@ __host__ __device__ inline int tix(int i, int j) { return i * (i + 1) / 2 + j; }
 struct Layout {
     int T, nL, nX;
     int fL, fD, fX, fF, fR, fC, ctl, nsync;
-    int nblocks;
+    int nblocks;  // without the refinement's 3 T
     size_t oL, oX, oT, oW, oA, oS, oDS, oP, oSc, nws;  // workspace offsets (doubles)
 };
 
@@ -108,13 +127,14 @@ __host__ __device__ inline int lflag(const Layout& g, int i, int j) {
 }
 
 struct StepArgs {
-    int k, typ, ldg, do_adam;
+    int k, typ, ldg, do_adam, refine;
     double n_rows, M, lr, b1, b2, eps;
     const double* lam;
     const double* G;
     const double* b;
     const double* yy;
-    const double* c;  // y = Phi c + e with Phi^T e = 0, yy = |e|^2; or NULL
+    const double* c;  // y = Phi c + e, yy = |e|^2; or NULL
+    const double* g;  // Phi^T e
     const double* lower;
     double* u;
     const int* trainable;
@@ -384,6 +404,21 @@ __device__ dbl4 a_quadrant(const StepArgs& a, int i, int j, int qi, int qj, int 
     return v;
 }
 
+// l = C D^T, a panel tile's quadrant by the explicit inverse D of its diagonal
+// tile L, corrected by the residual: l += (C - l L^T) D^T, as exact as a solve
+// with L (the factor's residual without it: 1e-11 of A where cond(L) = 4e4).  C
+// is overwritten, tmp is another LDS tile.
+__device__ __forceinline__ void correct_panel(dbl4& l, double* C, double* tmp, const double* L, int ldl,
+                                              const double* D, int ldd, int qi, int qj, int lane) {
+    quad_store(l, tmp, LDT, qi, qj, lane);
+    __syncthreads();
+    dbl4 r = quad_load(C, LDT, qi, qj, lane);
+    tile_mma<true>(r, tmp, LDT, L, ldl, -1.0, qi, qj, lane);
+    quad_store(r, C, LDT, qi, qj, lane);
+    __syncthreads();
+    tile_mma<true>(l, C, LDT, D, ldd, 1.0, qi, qj, lane);
+}
+
 __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, double* lds) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int qi = wv >> 1, qj = wv & 1, T = g.T;
@@ -394,6 +429,7 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
     double* Cs = lds;                            // 32 x 33 (then L, D, scratch)
     double* dadd = lds + 4 * TB * LDT + 16 * 17;  // 32
     double* sh = dadd + TB;                       // 4
+    double* adiag = sh + 4;                       // 32, then whether the tile is ill
     // theta and the filter normalisation sum over all k eigenvalues
     const double nu = softplus_d(a.u[0]) + a.lower[0];
     const double kappa = softplus_d(a.u[1]) + a.lower[1];
@@ -408,13 +444,15 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
     sr = block_sum(sr, sh);
     if (tid < TB) {
         const int row = j * TB + tid;
-        double add = 0.0;
+        double add = 0.0, diag = 1.0;
         if (row < a.k) {
             double r, dn, dk;
             filter_terms(a.typ, a.lam[row], nu, kappa, r, dn, dk);
             add = s2 / fmax(sf * a.n_rows * r / sr, kMinS);
         }
+        if (row < a.k) diag = a.G[(size_t)row * a.ldg + row] + add;
         dadd[tid] = add;
+        adiag[tid] = diag;
     }
     __syncthreads();
     // C(j,j) and, below it, C(j+1,j): every update but C(j+1,j)'s last one
@@ -442,6 +480,11 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
     double* Ls = Cs + TB * LDT;  // 32 x 33: L(j,j)
     double* Ds = Ls + TB * LDT;  // 32 x 33: D(j) = L(j,j)^-1
     double* Ws = Ds + TB * LDT;  // 16 x 17 scratch
+    // the first n pivots kept too little of A's diagonal
+    auto ill = [&](int n) {
+        const double d = Ls[(lane & 31) * (LDT + 1)];
+        return a.refine && __any(lane < n && d * d < kIll * adiag[lane & 31]);
+    };
     if (wv == 0) {
         // upper-right 16 x 16 blocks of L and D are zero; the rest is written
         for (int e = lane; e < 256; e += 64) {
@@ -454,6 +497,13 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
         dbl4 t = mma16<true>(dbl4{0, 0, 0, 0}, Cs + 16 * LDT, LDT, Ds, LDT, 1.0, lane);  // C21 D11^T
         store16(t, Ls + 16 * LDT, LDT, lane);                                             // L21
         wave_lds_sync();
+        if (ill(16)) {  // L21 += (C21 - L21 L11^T) D11^T
+            store16(mma16<true>(load16(Cs + 16 * LDT, LDT, lane), Ls + 16 * LDT, LDT, Ls, LDT, -1.0, lane),
+                    Ws, 17, lane);
+            wave_lds_sync();
+            store16(mma16<true>(t, Ws, 17, Ds, LDT, 1.0, lane), Ls + 16 * LDT, LDT, lane);
+            wave_lds_sync();
+        }
         dbl4 c22 = load16(Cs + 16 * LDT + 16, LDT, lane);
         c22 = mma16<true>(c22, Ls + 16 * LDT, LDT, Ls + 16 * LDT, LDT, -1.0, lane);
         store16(c22, Ws, 17, lane);
@@ -468,6 +518,12 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
         wave_lds_sync();
         bad = (int)wave_max((double)bad);
         if (bad && lane == 0) atomicOr(ctl + 2, 1);
+        const bool lost = ill(32);
+        if (lane == 0) {
+            if (lost) atomicOr(ctl + 3, 1);
+            adiag[TB] = lost;
+            a.ws[g.oP + 8 * (size_t)j + 7] = lost;  // for the panel tasks; free until column j's sums
+        }
     } else if (has1 && j > 0) {
         // meanwhile waves 1-3 apply C(j+1,j)'s last update, from L(j+1,j-1),
         // quadrant by quadrant in LDS (wave 1: (0,0) and (1,1); wave 2: (0,1);
@@ -488,6 +544,7 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
         // L(j+1,j) = C(j+1,j) D(j)^T
         dbl4 l1 = dbl4{0, 0, 0, 0};
         tile_mma<true>(l1, C1, LDT, Ds, LDT, 1.0, qi, qj, lane);
+        if (adiag[TB] != 0.0) correct_panel(l1, C1, Cs, Ls, LDT, Ds, LDT, qi, qj, lane);
         quad_store(l1, Lt + (size_t)tix(j + 1, j) * TT, TB, qi, qj, lane);
     }
     {
@@ -521,7 +578,10 @@ __device__ void task_offdiag(const StepArgs& a, const Layout& g, int i, int j, i
     quad_store(acc, Cs, LDT, qi, qj, lane);
     wait_for(sync + g.fD + j, epoch, ctl);  // also orders the LDS stores above
     dbl4 l = dbl4{0, 0, 0, 0};
-    tile_mma<true>(l, Cs, LDT, Xt + (size_t)tix(j, j) * TT, TB, 1.0, qi, qj, lane);  // C D(j)^T
+    const double* D = Xt + (size_t)tix(j, j) * TT;
+    tile_mma<true>(l, Cs, LDT, D, TB, 1.0, qi, qj, lane);  // C D(j)^T
+    if (a.refine && a.ws[g.oP + 8 * (size_t)j + 7] != 0.0)
+        correct_panel(l, Cs, Cs + TB * LDT, Lt + (size_t)tix(j, j) * TT, TB, D, TB, qi, qj, lane);
     quad_store(l, Lt + (size_t)tix(i, j) * TT, TB, qi, qj, lane);
     publish(sync + lflag(g, i, j), epoch);
 }
@@ -587,56 +647,105 @@ __device__ void task_filter(const StepArgs& a, const Layout& g, int epoch, doubl
     publish(a.sync + g.fF, epoch);
 }
 
+// Whether this step refines: known when the last row has seen every diagonal
+// tile.  (The final task clears the word, of a step that did not refine maybe
+// before every workgroup has read it; of one that did it waits for them.)
+__device__ bool refining(const StepArgs& a, const Layout& g, int epoch) {
+    wait_for(a.sync + g.fR + g.T - 1, epoch, a.sync + g.ctl);
+    return ld_flag(a.sync + g.ctl + 3) != 0;
+}
+
+// r_i = b_i - s2 w_i / S_i - sum_j G(i,j) w_j, from G as it is: the refinement
+// then corrects what the factor and its inverse lost.  t has been read by every
+// column: the residual takes its place.
+__device__ void task_residual(const StepArgs& a, const Layout& g, int i, int epoch) {
+    if (!refining(a, g, epoch)) return;
+    const int tid = threadIdx.x, T = g.T, k = a.k;
+    int* sync = a.sync;
+    const int r = tid >> 3, q = tid & 7, row = i * TB + r;
+    const double* wv = a.ws + g.oW;
+    wait_all([&](int j) { return j < T ? sync + g.fC + j : sync + g.fF; }, T + 1, epoch, sync + g.ctl);
+    double s = 0.0;
+    if (row < k)
+        for (int j = 0; j < T; ++j)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int col = j * TB + 4 * q + c;
+                if (col < k) s += a.G[(size_t)row * a.ldg + col] * wv[col];
+            }
+    s += __shfl_xor(s, 1, 64);
+    s += __shfl_xor(s, 2, 64);
+    s += __shfl_xor(s, 4, 64);
+    if (q == 0) {
+        double res = 0.0;
+        if (row < k) {
+            const double s2 = softplus_d(a.u[3]) + a.lower[3];
+            res = a.b[row] - s2 * (wv[row] / a.ws[g.oS + row]) - s;
+        }
+        a.ws[g.oT + row] = res;
+    }
+    publish(sync + g.fR + i, epoch + 1);
+}
+
 // t_i = sum_{j<=i} X(i,j) b_j, tile by tile as the X tiles arrive: thread
 // (r = tid/8, q = tid%8) takes row r, columns 4q..4q+3 of every tile, then
-// the 8 partial sums meet by shuffles
-__device__ void task_row(const StepArgs& a, const Layout& g, int i, int epoch) {
+// the 8 partial sums meet by shuffles.  second: of the residual in b's place,
+// into the array that the columns then do without.
+__device__ void task_row(const StepArgs& a, const Layout& g, int i, int epoch, bool second) {
     const int tid = threadIdx.x, T = g.T;
     int* sync = a.sync;
     int* ctl = sync + g.ctl;
+    if (second && !refining(a, g, epoch)) return;
     const double* Xt = a.ws + g.oX;
     const int r = tid >> 3, q = tid & 7;
     double s = 0.0;
+    const double* b = second ? a.ws + g.oT : a.b;
     // every X(i, .) tile follows D(i) within a hand-off or two: wait for the
-    // whole row at once
-    wait_all([&](int j) { return j == i ? sync + g.fD + i : sync + g.fX + xid(T, i, j); }, i + 1,
-             epoch, ctl);
+    // whole row at once (the residuals come after all of them)
+    wait_all([&](int j) { return second ? sync + g.fR + j : j == i ? sync + g.fD + i : sync + g.fX + xid(T, i, j); },
+             i + 1, second ? epoch + 1 : epoch, ctl);
     for (int j = 0; j <= i; ++j) {
         const double* X = Xt + (size_t)tix(i, j) * TT + r * TB + 4 * q;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const int col = j * TB + 4 * q + c;
-            s += X[c] * (col < a.k ? a.b[col] : 0.0);
+            s += X[c] * (col < a.k ? b[col] : 0.0);
         }
     }
     s += __shfl_xor(s, 1, 64);
     s += __shfl_xor(s, 2, 64);
     s += __shfl_xor(s, 4, 64);
-    if (q == 0) a.ws[g.oT + (size_t)i * TB + r] = s;
-    publish(sync + g.fR + i, epoch);
+    if (q == 0) a.ws[(second ? g.oA : g.oT) + (size_t)i * TB + r] = s;
+    publish(sync + g.fR + i, second ? epoch + 2 : epoch);
 }
 
 // Tile column j of w = X^T t and diag(A^-1) (thread (c = tid%32, q = tid/32)
 // takes column c, rows 4q..4q+3 of every tile; the 8 partials are summed in
-// q order), then this column's share of every sum the NLML and adjoint need:
+// q order); second: of the correction of w.  Then,
+// unless a refinement follows, this column's share of every sum the NLML and
+// adjoint need:
 //   P[0] = sum b_q w_q       P[1] = sum w_q^2 / S_q    P[2] = sum A^-1_qq / S_q
 //   P[3] = sum log L_qq      P[4..6] = sum gS_q dS_q/d(nu, kappa, sigma_f)
 // with gS_q = (1/S_q - s2 A^-1_qq / S_q^2 - w_q^2 / S_q^2) / 2.
-// With the split y = Phi c + e, Phi^T e = 0 (a.c), p_q = w_q / S_q is
-// (Phi^T K_y^-1 y)_q and the first two become
-//   P[0] = sum c_q p_q          (y^T K_y^-1 y = P[0] + |e|^2 / s2)
-//   P[1] = sum p_q (c_q - w_q) / s2   (|K_y^-1 y|^2 = P[1] + |e|^2 / s2^2),
-// where y^T y - b^T w of the other form cancels to s2 times its terms.
-__device__ void task_col(const StepArgs& a, const Layout& g, int j, int epoch, double* lds) {
+// With a split y = Phi c + e (a.c) and g = Phi^T e (a.g), p_q = w_q / S_q is
+// (Phi^T K_y^-1 y)_q, the first two become
+//   P[0] = sum c_q p_q                P[1] = sum p_q (c_q - w_q) / s2
+// and P[7] = sum g_q (c_q - w_q): with t = |e|^2 + P[7],
+//   y^T K_y^-1 y = P[0] + t / s2,     |K_y^-1 y|^2 = P[1] + t / s2^2,
+// where y^T y - b^T w of the other form cancels to s2 times its terms.  Both
+// hold for any c; P[7] is the part of y in directions of Phi that the split
+// left in e.
+__device__ void task_col(const StepArgs& a, const Layout& g, int j, int epoch, double* lds, bool second) {
     const int tid = threadIdx.x, T = g.T, k = a.k;
     int* sync = a.sync;
     int* ctl = sync + g.ctl;
+    if (second && !refining(a, g, epoch)) return;
     const double* Xt = a.ws + g.oX;
-    const double* tv = a.ws + g.oT;
+    const double* tv = a.ws + (second ? g.oA : g.oT);
     const int c = tid & 31, q = tid >> 5;
     double sw = 0.0, sa = 0.0;
     for (int i = j; i < T; ++i) {
-        wait_for(sync + g.fR + i, epoch, ctl);  // row i has seen every X(i, .)
+        wait_for(sync + g.fR + i, second ? epoch + 2 : epoch, ctl);  // row i has seen every X(i, .)
         const double* X = Xt + (size_t)tix(i, j) * TT;
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
@@ -646,12 +755,13 @@ __device__ void task_col(const StepArgs& a, const Layout& g, int j, int epoch, d
             sa += x * x;
         }
     }
+    const bool more = a.refine && ld_flag(ctl + 3) != 0;  // the last row is there (refining())
     double* pw = lds;            // 8 x 32
     double* pa = lds + 8 * TB;   // 8 x 32
     pw[q * TB + c] = sw;
     pa[q * TB + c] = sa;
     wait_for(sync + g.fF, epoch, ctl);  // S, dS (also orders the LDS stores)
-    double v[7] = {0, 0, 0, 0, 0, 0, 0};
+    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (tid < TB) {
         const int qq = j * TB + tid;
         double w = 0.0, av = 0.0;
@@ -660,16 +770,24 @@ __device__ void task_col(const StepArgs& a, const Layout& g, int j, int epoch, d
             w += pw[h * TB + tid];
             av += pa[h * TB + tid];
         }
+        if (second) w += a.ws[g.oW + qq];
         a.ws[g.oW + qq] = w;
-        a.ws[g.oA + qq] = av;
-        if (qq < k) {
+        if (!more) a.ws[g.oA + qq] = av;
+        if (qq < k && (second || !more)) {
             const double s2 = softplus_d(a.u[3]) + a.lower[3];
             const double S = a.ws[g.oS + qq];
             const double* dS = a.ws + g.oDS;
             const double p = w / S;
             const double gS = 0.5 * ((1.0 - s2 * av / S) / S - p * p);
-            v[0] = a.c != nullptr ? a.c[qq] * p : a.b[qq] * w;
-            v[1] = a.c != nullptr ? p * ((a.c[qq] - w) / s2) : w * p;
+            if (a.c != nullptr) {
+                const double d = a.c[qq] - w;
+                v[0] = a.c[qq] * p;
+                v[1] = p * (d / s2);
+                v[7] = a.g[qq] * d;
+            } else {
+                v[0] = a.b[qq] * w;
+                v[1] = w * p;
+            }
             v[2] = av / S;
             v[3] = log(a.ws[g.oL + (size_t)tix(j, j) * TT + tid * TB + tid]);
             v[4] = gS * dS[qq];
@@ -679,12 +797,12 @@ __device__ void task_col(const StepArgs& a, const Layout& g, int j, int epoch, d
     }
     if (tid < 64) {  // wave 0: lanes 32..63 carry zeros
 #pragma unroll
-        for (int m = 0; m < 7; ++m) v[m] = wave_sum(v[m]);
+        for (int m = 0; m < 8; ++m) v[m] = wave_sum(v[m]);
         if (tid == 0)
 #pragma unroll
-            for (int m = 0; m < 7; ++m) a.ws[g.oP + 8 * (size_t)j + m] = v[m];
+            for (int m = 0; m < 8; ++m) a.ws[g.oP + 8 * (size_t)j + m] = v[m];
     }
-    publish(sync + g.fC + j, epoch);
+    publish(sync + g.fC + j, a.refine && second == more ? epoch + 1 : epoch);  // the sums are there
 }
 
 // NLML and adjoint (gp.hip's weight-space finish, one right-hand side, with
@@ -696,22 +814,24 @@ __device__ void task_final(const StepArgs& a, const Layout& g, int epoch) {
     int* ctl = sync + g.ctl;
     // the column tasks all finish after the last row: wait for them (and the
     // filter) at once
-    wait_all([&](int j) { return j < T ? sync + g.fC + j : sync + g.fF; }, T + 1, epoch, ctl);
+    wait_all([&](int j) { return j < T ? sync + g.fC + j : sync + g.fF; }, a.refine ? T : T + 1,
+             a.refine ? epoch + 1 : epoch, ctl);
     if (tid < 4) {
         const int p = tid;
-        double P[7] = {0, 0, 0, 0, 0, 0, 0};
+        double P[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         for (int j = 0; j < T; ++j)
 #pragma unroll
-            for (int m = 0; m < 7; ++m) P[m] += a.ws[g.oP + 8 * (size_t)j + m];
+            for (int m = 0; m < 8; ++m) P[m] += a.ws[g.oP + 8 * (size_t)j + m];
         const double bw = P[0], ww = P[1], tr = P[2], ld = P[3];
         const double lS = a.ws[g.oSc];
         const double s2 = softplus_d(a.u[3]) + a.lower[3];
         const double y2 = a.yy[0], M = a.M;
         const double two_pi = 6.283185307179586;
         // y^T K_y^-1 y and |K_y^-1 y|^2
-        const double ya = a.c != nullptr ? bw + y2 / s2 : (y2 - bw) / s2;
+        const double t2 = y2 + P[7];
+        const double ya = a.c != nullptr ? bw + t2 / s2 : (y2 - bw) / s2;
         const double wGw = bw - s2 * ww;
-        const double aa = a.c != nullptr ? ww + y2 / (s2 * s2) : (y2 - 2.0 * bw + wGw) / (s2 * s2);
+        const double aa = a.c != nullptr ? ww + t2 / (s2 * s2) : (y2 - 2.0 * bw + wGw) / (s2 * s2);
         const double nlml = 0.5 * ya + 0.5 * ((M - k) * log(s2) + lS + 2.0 * ld) +
                             0.5 * M * log(two_pi);
         const double gs2 = 0.5 * ((M - k) / s2 + tr - aa);
@@ -742,12 +862,13 @@ __device__ void task_final(const StepArgs& a, const Layout& g, int epoch) {
         a.status[0] = err ? RVGP_ST_TIMEOUT : (nspd ? RVGP_ST_NOT_SPD : RVGP_ST_OK);
         st_flag(ctl + 1, 0);
         st_flag(ctl + 2, 0);
-        st_flag(ctl, epoch);  // the next launch runs epoch + 1
+        st_flag(ctl + 3, 0);
+        st_flag(ctl, a.refine ? epoch + 2 : epoch);  // the next launch runs one more
     }
 }
 
 __global__ __launch_bounds__(NTH) void ws_step_kernel(StepArgs a) {
-    __shared__ double lds[4 * TB * LDT + 16 * 17 + 64];
+    __shared__ double lds[4 * TB * LDT + 16 * 17 + 72];
     __shared__ int s_epoch;
     const Layout g = make_layout(a.k);
     // the previous launch's final task stored the epoch; every task reads it
@@ -777,9 +898,13 @@ __global__ __launch_bounds__(NTH) void ws_step_kernel(StepArgs a) {
     b -= g.nX;
     if (b == 0) { task_filter(a, g, epoch, lds); return; }
     b -= 1;
-    if (b < T) { task_row(a, g, b, epoch); return; }
+    if (b < T) { task_row(a, g, b, epoch, false); return; }
     b -= T;
-    if (b < T) { task_col(a, g, b, epoch, lds); return; }
+    if (b < T) { task_col(a, g, b, epoch, lds, false); return; }
+    b -= T;
+    if (a.refine && b < T) { task_residual(a, g, b, epoch); return; }
+    if (a.refine && b < 2 * T) { task_row(a, g, b - T, epoch, true); return; }
+    if (a.refine && b < 3 * T) { task_col(a, g, b - 2 * T, epoch, lds, true); return; }
     task_final(a, g, epoch);
 }
 
@@ -798,7 +923,7 @@ extern "C" size_t rvgp_ws_step_sync_ints(int k) {
     return (size_t)make_layout(k).nsync;
 }
 
-static int ws_step(const double* c, int k, int typ, const double* evals, double n_rows, const double* G,
+static int ws_step(const double* c, const double* ge, int k, int typ, const double* evals, double n_rows, const double* G,
                    int ldg, const double* b, const double* yy, double M, const double* lower,
                    double* u, const int* trainable, double* m1, double* m2, double* t, int do_adam,
                    double lr, double b1, double b2, double eps, void* ws, size_t ws_bytes, int* sync,
@@ -817,7 +942,11 @@ static int ws_step(const double* c, int k, int typ, const double* evals, double 
     a.typ = typ;
     a.ldg = ldg;
     a.do_adam = do_adam;
+    // a host optimiser's evaluations and the split form; an Adam step of the
+    // weight form, whose y^T y - b^T w loses as much, does without
+    a.refine = c != nullptr || !do_adam;
     a.c = c;
+    a.g = ge;
     a.n_rows = n_rows;
     a.M = M;
     a.lr = lr;
@@ -838,7 +967,8 @@ static int ws_step(const double* c, int k, int typ, const double* evals, double 
     a.sync = sync;
     a.out = out;
     a.status = status;
-    hipLaunchKernelGGL(ws_step_kernel, dim3(g.nblocks), dim3(NTH), 0, as_stream(stream), a);
+    hipLaunchKernelGGL(ws_step_kernel, dim3(g.nblocks + (a.refine ? 3 * g.T : 0)), dim3(NTH), 0,
+                       as_stream(stream), a);
     RVGP_LAUNCH_CHECK();
     return RVGP_OK;
 }
@@ -849,17 +979,17 @@ extern "C" int rvgp_ws_step(int k, int typ, const double* evals, double n_rows, 
                             double* m2, double* t, int do_adam, double lr, double b1, double b2,
                             double eps, void* ws, size_t ws_bytes, int* sync, size_t sync_ints,
                             double* out, int* status, void* stream) {
-    return ws_step(nullptr, k, typ, evals, n_rows, G, ldg, b, yy, M, lower, u, trainable, m1, m2, t, do_adam,
+    return ws_step(nullptr, nullptr, k, typ, evals, n_rows, G, ldg, b, yy, M, lower, u, trainable, m1, m2, t, do_adam,
                    lr, b1, b2, eps, ws, ws_bytes, sync, sync_ints, out, status, stream);
 }
 
 extern "C" int rvgp_coef_step(int k, int typ, const double* evals, double n_rows, const double* G,
-                              int ldg, const double* b, const double* c, const double* ee,
+                              int ldg, const double* b, const double* c, const double* ge, const double* ee,
                               double M, const double* lower, double* u, const int* trainable, double* m1,
                               double* m2, double* t, int do_adam, double lr, double b1, double b2,
                               double eps, void* ws, size_t ws_bytes, int* sync, size_t sync_ints,
                               double* out, int* status, void* stream) {
-    RVGP_CHECK_ARG(c != nullptr, "rvgp_coef_step: c is NULL");
-    return ws_step(c, k, typ, evals, n_rows, G, ldg, b, ee, M, lower, u, trainable, m1, m2, t, do_adam,
+    RVGP_CHECK_ARG(c != nullptr && ge != nullptr, "rvgp_coef_step: c or ge is NULL");
+    return ws_step(c, ge, k, typ, evals, n_rows, G, ldg, b, ee, M, lower, u, trainable, m1, m2, t, do_adam,
                    lr, b1, b2, eps, ws, ws_bytes, sync, sync_ints, out, status, stream);
 }

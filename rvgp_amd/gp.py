@@ -8,12 +8,12 @@ Two exact forms of the same model y ~ N(0, Phi diag(S) Phi^T + s2 I):
   * function space: M x M Gram on the matrix cores (rvgp_gemm with the
     spectral filter as k-scale), blocked Cholesky, triangular solves;
     with at least twice as many rows as features (or in mixed precision) no
-    M x M matrix is formed: with y = Phi c + e, Phi^T e = 0, split once per
-    training set, and w of the FP64 k x k system below, p = Phi^T K_y^-1 y =
-    w / S, y^T K_y^-1 y = c^T p + |e|^2 / s2 and |K_y^-1 y|^2 = p^T (c - w) / s2
-    + |e|^2 / s2^2, without the weight form's y^T y - b^T w, which cancels at
-    small noise; a mixed fit with fewer rows solves by Woodbury, refined
-    against the matrix-free FP64 K_y.
+    M x M matrix is formed: with y = Phi c + e, split once per training set,
+    g = Phi^T e, w of the FP64 k x k system below and t = |e|^2 + g^T (c - w),
+    p = Phi^T K_y^-1 y = w / S, y^T K_y^-1 y = c^T p + t / s2 and |K_y^-1 y|^2 =
+    p^T (c - w) / s2 + t / s2^2 for any c, without the weight form's
+    y^T y - b^T w, which cancels at small noise; a mixed fit with fewer rows
+    solves by Woodbury, refined against the matrix-free FP64 K_y.
   * weight space (Woodbury / determinant lemma): k x k system
     A = s2 S^-1 + Phi^T Phi; G = Phi^T Phi and b = Phi^T y are formed once per
     training set, so an optimiser step costs O(k^3) and never touches an
@@ -87,13 +87,21 @@ FUSED_STEP_MAX_K = 2048  # RVGP_WS_STEP_MAX_K
 # A function-space fit of M rows works on the k x k system from M = 2 k on.
 # Its flops are ~(k / M)^3 of the M x M factorisation's; below 2 k rows
 # Phi^T Phi is singular for the tangent fields' frames (rank m d < M).
-# M = 4731, k = 200: an evaluation 10.0 -> 0.14 ms, building the engine 0.84 ms.
-# Its error against 80-bit arithmetic, noise 1 ... 1e-6, data with noise: NLML
-# <= 4e-13 and gradient <= 5e-13 (M x M: 1e-8 and 3e-8), mean 2e-13 (7e-8),
-# variance 1e-13 (5e-7); without noise, s2 -> 1e-6: gradient 1e-9 (2e-12), the
-# others as before or better.
+# M = 4731, k = 200: an evaluation 10.0 -> 0.09 ms (0.11 ms where Phi^T Phi is
+# close to singular and the step refines), building the engine 0.97 ms.
+# Its error against 80-bit arithmetic, in brackets the M x M form's, on Fourier
+# columns (M = 300, k = 40) with noise 0.05, s2 = 0.1 ... 2e-6.  Nodes all over the
+# circle: NLML 6e-14 ... 9e-11 (3e-11 ... 4e-3), gradient <= 3e-15 of its largest
+# entry (6e-8).  On half of it, where Phi^T Phi is singular to working precision:
+# 7e-11 ... 2e-4 (2e-11 ... 6e-3) and <= 2e-9 (8e-8).  What it is worse at: such a
+# Phi^T Phi with data without noise, whose rounding in the null space counts
+# against s2 / S: NLML 7e-11 ... 3e-6 (3e-11 ... 8e-7), gradient <= 2e-8 (1e-10).
 COEF_MIN_ROWS = 2
-SPLIT_RIDGE = 1e-12  # of the largest diagonal entry of Phi^T Phi
+# The ridge of the split, of the largest diagonal entry of Phi^T Phi: small
+# enough that little is left in e, large enough that c stays small in
+# directions where Phi^T Phi is rounding (1e-12: rounding of Phi c up to 3e-4 in
+# the NLML at s2 = 1e-6, 1e-6: 8e-4 from what is left; 1e-9: the least of both).
+SPLIT_RIDGE = 1e-9
 
 
 class GPREngine:
@@ -207,25 +215,27 @@ class GPREngine:
                                       device=self.dev)
 
     def _split_rows(self):
-        """y = Phi c + e with Phi^T e = 0: c (k, R) and |e|^2, by the Cholesky
-        factor of G with a ridge, three passes against the rows.  Duplicated
-        features and fewer tangent rows than features leave G singular: the
-        ridge makes it solvable, the passes take the ridge's share out of every
-        direction the rows hold, and any c with the right Phi c serves.  False
+        """y = Phi c + e: c (k, R), |e|^2 and g = Phi^T e (k, R), by the Cholesky
+        factor of G with a ridge, two passes against the rows.  Duplicated
+        features, fewer tangent rows than features and nodes on a part of the
+        manifold leave G singular: the ridge makes it solvable, and what it
+        leaves in e of directions that the rows hold, g accounts for.  False
         when G is not positive definite even so."""
         L = self.G + (SPLIT_RIDGE * torch.diagonal(self.G).max()) * torch.eye(
             self.k, dtype=torch.float64, device=self.dev)
         _, st = dense.potrf(L, check=False)
         if int(st.item()) != 0:
             return False
-        c, e = torch.zeros_like(self.b), self.y
-        for _ in range(3):
-            r = dense.gemm(self.Phi, e, transA=True)
+        c, g = torch.zeros_like(self.b), self.b
+        for _ in range(2):
+            r = g.clone()
             dense.trsm(L, r)
             dense.trsm(L, r, trans=True)
             c = c + r
             e = (self.y - dense.gemm(self.Phi, c)).contiguous()
-        self.c, self.ee = c.contiguous(), torch.empty(1, dtype=torch.float64, device=self.dev)
+            g = dense.gemm(self.Phi, e, transA=True)
+        self.c, self.g = c.contiguous(), g
+        self.ee = torch.empty(1, dtype=torch.float64, device=self.dev)
         self._dot(e, e, self.ee)
         return True
 
@@ -291,7 +301,7 @@ class GPREngine:
     def evaluate(self):
         """Enqueue NLML + gradient; results in self.out (device):
         [nlml, d/d(nu, kappa, sigma_f, s2), d/du(...)].  One launch where the
-        single-launch step serves the fit (k = 500: 216 against 358 us)."""
+        single-launch step serves the fit (k = 500: 185 against 356 us)."""
         return self._ws_step(0) if self.fused() else self._evaluate_state()
 
     def _evaluate_state(self):
@@ -313,6 +323,11 @@ class GPREngine:
             self._colsumsq(self.Linv, self.ainv)
             t = dense.gemm(self.Linv, self.b)
             dense.gemm(self.Linv, t, self.w, transA=True)
+            if self.coef:
+                # one refinement: L^-1 is good to cond(L), a solve with L to less
+                r = self.b - self.s2 * (self.w / self.S.reshape(-1, 1))
+                dense.gemm(self.G, self.w, r, alpha=-1.0, beta=1.0)
+                dense.gemm(self.Linv, dense.gemm(self.Linv, r), self.w, transA=True, beta=1.0)
         if self.form == "weight":
             Gw = dense.gemm(self.G, self.w)
             _lib.call("rvgp_ws_finish", self.k, float(self.M), self.R, _lib.ptr(self.A), self.k,
@@ -322,10 +337,10 @@ class GPREngine:
             return self.out
         if self.coef:
             p = (self.w / self.S.reshape(-1, 1)).contiguous()  # Phi^T K_y^-1 y
-            self._dot(self.c, p, self.ya)
-            self._dot(p, ((self.c - self.w) / self.s2).contiguous(), self.aa)
-            self.ya += self.ee / self.s2
-            self.aa += self.ee / (self.s2 * self.s2)
+            d = (self.c - self.w).contiguous()
+            t = (self._dot(self.g, d, torch.empty_like(self.ee)) + self.ee) / self.s2
+            self._dot(self.c, p, self.ya).add_(t)
+            self._dot(p, d, self.aa).add_(t).div_(self.s2)
         elif self.precision == "mixed":
             # alpha = K_y^-1 y = (y - Phi w) / s2 (Woodbury; w = A^-1 Phi^T y
             # above), then two refinement sweeps against the FP64 K_y
@@ -487,7 +502,7 @@ class GPREngine:
         args = (_lib.ptr(self.m1), _lib.ptr(self.m2), _lib.ptr(self.t),
                 _lib.ptr(self.trainable)) if do_adam else (None, None, None, None)
         m1, m2, t, tr = args
-        y = (self.b, self.c, self.ee) if self.coef else (self.b, self.yy)
+        y = (self.b, self.c, self.g, self.ee) if self.coef else (self.b, self.yy)
         _lib.call("rvgp_coef_step" if self.coef else "rvgp_ws_step", self.k, self.typ,
                   _lib.ptr(self.evals), self.n_rows, _lib.ptr(self.G), self.G.stride(0),
                   *[_lib.ptr(t) for t in y],

@@ -64,3 +64,74 @@ def test_trial_steps_far_out_stay_finite():
         s2 = np.log1p(np.exp(u[3])) + 1e-6
         noise = 0.5 * float((y * y).sum()) / s2 + 60.0 * np.log(2 * np.pi * s2)
         assert np.isfinite(v) and np.all(np.isfinite(g)) and v == pytest.approx(noise, rel=1e-6)
+
+
+def _extended(Phi, y, lam, th, n_rows):
+    """NLML and its gradient in 80 bits: in an orthonormal basis of the rows,
+    Phi = Q T, y = Q a + e, the covariance acts as T S T^T + s2 I on a and as s2 on e."""
+    X = np.longdouble
+    Phi, y, lam = Phi.astype(X), y.astype(X), lam.astype(X)
+    nu, kappa, sf, s2 = (X(v) for v in th)
+    M, k = Phi.shape
+    Q, T = np.zeros((M, k), X), np.zeros((k, k), X)
+    for j in range(k):
+        v = Phi[:, j].copy()
+        for _ in range(3):
+            h = Q[:, :j].T @ v
+            v, T[:j, j] = v - Q[:, :j] @ h, T[:j, j] + h
+        T[j, j] = np.sqrt(v @ v)
+        Q[:, j] = v / T[j, j]
+    a = Q.T @ y
+    e = y - Q @ a
+    base = lam + 2 * nu / kappa ** 2
+    r = base ** -nu
+    dn, dk = -np.log(base) - nu * (2 / kappa ** 2) / base, 4 * nu ** 2 / (kappa ** 3 * base)
+    S = sf * X(n_rows) * r / r.sum()
+    dS = np.stack([S * (dn - r @ dn / r.sum()), S * (dk - r @ dk / r.sum()), S / sf])
+    L = (T * S) @ T.T + s2 * np.eye(k, dtype=X)
+    for j in range(k):
+        L[j:, j] /= np.sqrt(L[j, j])
+        L[j + 1:, j + 1:] -= np.outer(L[j + 1:, j], L[j + 1:, j])
+    L = np.tril(L)
+
+    def solve(B):
+        B = B.copy()
+        for i in range(k):
+            B[i] = (B[i] - L[i, :i] @ B[:i]) / L[i, i]
+        return B
+
+    Li = solve(np.eye(k, dtype=X))
+    z, q = Li @ a, ((Li @ T) ** 2).sum(0)
+    p, rhs = T.T @ (Li.T @ z), y.shape[1]
+    logdet = 2 * np.log(np.diag(L)).sum() + (M - k) * np.log(s2)
+    nlml = ((z * z).sum() + (e * e).sum() / s2 + rhs * (logdet + M * np.log(2 * X(np.pi)))) / 2
+    alpha2 = ((Li.T @ z) ** 2).sum() + (e * e).sum() / s2 ** 2
+    grad = np.append(dS @ (rhs * q - (p * p).sum(1)), rhs * (M - S @ q) / s2 - alpha2) / 2
+    return float(nlml), grad.astype(float), S.astype(float)
+
+
+# nodes on a part of a circle: the columns are close to dependent, with singular
+# values of every size down to rounding
+@pytest.mark.parametrize("M,k,part", [(300, 40, 0.5), (240, 60, 0.33)])
+@pytest.mark.parametrize("R", [1, 3])
+@pytest.mark.parametrize("noise", [0.05, 1e-3])
+@pytest.mark.parametrize("s2", [1e-1, 2.5e-3, 1e-4, 2e-6])
+def test_nodes_on_a_part_of_the_manifold(M, k, part, R, noise, s2):
+    rng = np.random.default_rng(k)
+    t, f = 2 * np.pi * part * rng.uniform(size=(M, 1)), np.arange(1, k) // 2 + np.arange(1, k) % 2
+    Phi = np.concatenate([np.ones((M, 1)), np.sqrt(2) * np.where(np.arange(1, k) % 2, np.cos(f * t), np.sin(f * t))], 1)
+    lam = 0.05 * np.append(0, f) ** 2.0
+    y = Phi @ (rng.normal(size=(k, R)) / (1 + 5 * lam[:, None]))
+    y = y / np.abs(y).max() + noise * rng.normal(size=(M, R))
+    e = _engine(Phi, y, lam)
+    th = (1.6, 4.0, 0.8, s2)
+    e.set_theta(th)
+    assert e.coef
+    nlml, _, out = e.nlml_grad_u(e.u.cpu().numpy())
+    ref, grad, S = _extended(Phi, y, lam, th, 500.0)
+    # rounding of Phi c, where |c| <= |y| / sqrt(ridge G), and of G, against s2; two
+    # passes of two products
+    off = 4 * np.finfo(float).eps * ((y * y).sum() / np.sqrt(1e-9) + R * (Phi * Phi).sum(0) @ S) / s2
+    assert abs(nlml - ref) <= off + 1e-9 * abs(ref)
+    np.testing.assert_allclose(out[1:4], grad[:3], rtol=1e-7, atol=10 * off)
+    np.testing.assert_allclose(out[4], grad[3], rtol=1e-9, atol=off / s2)
