@@ -366,6 +366,11 @@ int rvgp_colsumsq_noalloc(int f64, int M, int k, const void* Z, int ldz, double*
 int rvgp_spectral_filter(int typ, int k, const double* evals, const double* theta, double n_rows,
                          double* S, double* dS, void* stream);
 
+/* rvgp_spectral_filter for a system that divides by S (rvgp_ws_form): values
+ * below 1e-280 are raised to it, a NaN stays one. */
+int rvgp_system_filter(int typ, int k, const double* evals, const double* theta, double n_rows,
+                       double* S, double* dS, void* stream);
+
 /* A = G + diag(s2 / S)  (weight-space system matrix), s2 a device scalar. */
 int rvgp_ws_form(int k, const double* G, int ldg, const double* S, const double* s2, double* A,
                  int lda, void* stream);

@@ -38,6 +38,11 @@ static inline size_t align_up(size_t a, size_t b) { return (a + b - 1) / b * b; 
 
 constexpr int kWave = 64;
 
+// Filter values that an optimiser's trial step sends to 0 (a sigma_f of 1e-300, a
+// steep filter) are raised to this where 1 / S is taken: it stays finite, S
+// itself is as good as 0.
+constexpr double kMinFilter = 1e-280;
+
 // Wave-wide reductions via cross-lane shuffles.
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {

@@ -45,11 +45,13 @@ __device__ double block_sum(double v, double* sh) {
     return s;
 }
 
-// theta = [nu, kappa, sigma_f]; S (k), dS (3, k)
+// theta = [nu, kappa, sigma_f]; S (k), dS (3, k).  S is at least `least` (NaN stays
+// NaN).
 __global__ __launch_bounds__(FT) void spectral_filter_kernel(int typ, int k,
                                                              const double* __restrict__ lam,
                                                              const double* __restrict__ theta,
-                                                             double n_rows, double* __restrict__ S,
+                                                             double n_rows, double least,
+                                                             double* __restrict__ S,
                                                              double* __restrict__ dS) {
     __shared__ double sh[FT / 64];
     const double nu = theta[0], kappa = theta[1], sf = theta[2];
@@ -86,7 +88,8 @@ __global__ __launch_bounds__(FT) void spectral_filter_kernel(int typ, int k,
             dn = 0.0;
             dk = -lam[j] * kappa;
         }
-        const double s = sf * n_rows * r / sr;
+        double s = sf * n_rows * r / sr;
+        s = s < least ? least : s;
         S[j] = s;
         if (dS) {
             dS[j] = s * (dn - snu);
@@ -254,19 +257,19 @@ __global__ __launch_bounds__(FT) void ws_finish_kernel(int k, double M, int R,
     const double Rd = (double)R;
     double bw = 0.0, wGw = 0.0, ld = 0.0, lS = 0.0, tr = 0.0;
     for (int j = threadIdx.x; j < k; j += FT) {
-        double ww = 0.0;
+        const double sj = S[j];
+        double pp = 0.0;  // |w_j / S_j|^2, in this order: S_j^2 may underflow
         for (int r = 0; r < R; ++r) {
             const size_t e = (size_t)j * R + r;
             bw += b[e] * w[e];
             wGw += w[e] * Gw[e];
-            ww += w[e] * w[e];
+            pp += (w[e] / sj) * (w[e] / sj);
         }
         ld += log(L[(size_t)j * ldl + j]);
-        lS += log(S[j]);
+        lS += log(sj);
         const double ainv = ainv_diag[j];  // (A^-1)_jj = sum_i (L^-1)_ij^2
-        tr += ainv / S[j];
-        const double sj = S[j];
-        gS[j] = 0.5 * (Rd / sj - Rd * s2 * ainv / (sj * sj) - ww / (sj * sj));
+        tr += ainv / sj;
+        gS[j] = 0.5 * (Rd * (1.0 - s2 * ainv / sj) / sj - pp);
     }
     bw = block_sum(bw, sh);
     wGw = block_sum(wGw, sh);
@@ -371,14 +374,24 @@ __global__ void adam_kernel(double* __restrict__ u, const double* __restrict__ g
 
 using namespace rvgp;
 
-extern "C" int rvgp_spectral_filter(int typ, int k, const double* evals, const double* theta,
-                                    double n_rows, double* S, double* dS, void* stream) {
+static int spectral_filter(int typ, int k, const double* evals, const double* theta, double n_rows,
+                           double least, double* S, double* dS, void* stream) {
     RVGP_CHECK_ARG(typ == 0 || typ == 1, "rvgp_spectral_filter: typ must be 0 (matern) or 1 (se)");
     RVGP_CHECK_ARG(k >= 1, "rvgp_spectral_filter: k >= 1");
     hipLaunchKernelGGL(spectral_filter_kernel, dim3(1), dim3(FT), 0, as_stream(stream), typ, k, evals,
-                       theta, n_rows, S, dS);
+                       theta, n_rows, least, S, dS);
     RVGP_LAUNCH_CHECK();
     return RVGP_OK;
+}
+
+extern "C" int rvgp_spectral_filter(int typ, int k, const double* evals, const double* theta,
+                                    double n_rows, double* S, double* dS, void* stream) {
+    return spectral_filter(typ, k, evals, theta, n_rows, -__builtin_huge_val(), S, dS, stream);
+}
+
+extern "C" int rvgp_system_filter(int typ, int k, const double* evals, const double* theta,
+                                  double n_rows, double* S, double* dS, void* stream) {
+    return spectral_filter(typ, k, evals, theta, n_rows, kMinFilter, S, dS, stream);
 }
 
 extern "C" int rvgp_ws_form(int k, const double* G, int ldg, const double* S, const double* s2,
@@ -542,7 +555,7 @@ __global__ __launch_bounds__(256) void lemma_terms_kernel(int k, double M,
     double acc = 0.0;
     for (int j = threadIdx.x; j < k; j += 256) {
         const double sj = S[j];
-        q[j] = 1.0 / sj - s2 * ainv[j] / (sj * sj);
+        q[j] = (1.0 - s2 * ainv[j] / sj) / sj;  // S_j^2 may underflow
         acc += 0.5 * log(sj) + log(LA[(size_t)j * lda + j]);
     }
     acc = wave_sum(acc);

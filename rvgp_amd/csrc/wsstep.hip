@@ -66,9 +66,6 @@ constexpr int TT = TB * TB;     // doubles per tile
 constexpr int NTH = 256;        // threads per task workgroup (4 waves)
 constexpr int LDT = TB + 1;     // LDS tile row stride
 constexpr int kSpinLimit = 1 << 21;
-// Filter values that an optimiser's trial step sends to 0 (a sigma_f of 1e-300,
-// a steep filter): 1 / S stays finite, S itself is as good as 0.
-constexpr double kMinS = 1e-280;
 // L_qq^2 / A_qq below which explicit inverses lose more than a digit.  (At 1e-4
 // the NLML of 300 rows on half a circle, s2 = 1e-4, was off by 3e-5 unnoticed.)
 // Rows of nodes all over the manifold stay far above: such a step takes as long
@@ -382,6 +379,10 @@ __device__ __forceinline__ void filter_terms(int typ, double lam, double nu, dou
     }
 }
 
+// A filter value that 1 / S is taken of.  Not fmax, which drops a NaN (0 / 0 where
+// every r underflows): it has to reach the pivots and be reported.
+__device__ __forceinline__ double floored(double s) { return s < kMinFilter ? kMinFilter : s; }
+
 __device__ __forceinline__ double softplus_d(double x) {
     return x > 0 ? x + log1p(exp(-x)) : log1p(exp(x));
 }
@@ -448,7 +449,7 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
         if (row < a.k) {
             double r, dn, dk;
             filter_terms(a.typ, a.lam[row], nu, kappa, r, dn, dk);
-            add = s2 / fmax(sf * a.n_rows * r / sr, kMinS);
+            add = s2 / floored(sf * a.n_rows * r / sr);
         }
         if (row < a.k) diag = a.G[(size_t)row * a.ldg + row] + add;
         dadd[tid] = add;
@@ -635,7 +636,7 @@ __device__ void task_filter(const StepArgs& a, const Layout& g, int epoch, doubl
     for (int q = tid; q < k; q += NTH) {
         double r, dn, dk;
         filter_terms(a.typ, a.lam[q], nu, kappa, r, dn, dk);
-        const double v = fmax(sf * a.n_rows * r / sr, kMinS);
+        const double v = floored(sf * a.n_rows * r / sr);
         S[q] = v;
         dS[q] = v * (dn - snu);
         dS[k + q] = v * (dk - ska);

@@ -282,7 +282,9 @@ class GPREngine:
         s = _lib.stream()
         _lib.call("rvgp_gp_params", _lib.ptr(self.u), _lib.ptr(self.lower), _lib.ptr(self.theta),
                   _lib.ptr(self.s2), s)
-        _lib.call("rvgp_spectral_filter", self.typ, self.k, _lib.ptr(self.evals),
+        # the k x k system divides by S: the same floor as in the single-launch step
+        _lib.call("rvgp_system_filter" if self.normal else "rvgp_spectral_filter", self.typ, self.k,
+                  _lib.ptr(self.evals),
                   _lib.ptr(self.theta), self.n_rows, _lib.ptr(self.S), _lib.ptr(self.dS), s)
 
     def _dot(self, x, y, out):
@@ -311,8 +313,6 @@ class GPREngine:
         s = _lib.stream()
         self.status.zero_()
         if self.normal:
-            if self.coef:
-                self.S.clamp_(min=1e-280)  # a filter value of 0: 1 / S stays finite
             _lib.call("rvgp_ws_form", self.k, _lib.ptr(self.G), self.k, _lib.ptr(self.S),
                       _lib.ptr(self.s2), _lib.ptr(self.A), self.k, s)
             _lib.call("rvgp_potrf", 1, self.k, _lib.ptr(self.A), self.k, _lib.ptr(self.status), s)
