@@ -401,13 +401,22 @@ class GPREngine:
         """Differentiable NLML at x (see NLMLFunction)."""
         return NLMLFunction.apply(x, self, unconstrained)
 
+    def _read_result(self):
+        res = self._result.cpu()
+        return res, int(res[9:].view(torch.int32)[0])
+
     # ---------------------------------------------------------------- host API
     def nlml_grad_u(self, u):
         self.u.copy_(torch.from_numpy(np.array(u, np.float64)))
         self.evaluate()
-        res = self._result.cpu()
+        res, status = self._read_result()
+        if status == _lib.ST_TIMEOUT:
+            # a wait between workgroups of the single-launch step gave up (a GPU
+            # taken by other work): the launch-by-launch form waits for nothing
+            self._evaluate_state()
+            res, status = self._read_result()
         out = res[:9].numpy()
-        if int(res[9:].view(torch.int32)[0]) != 0:
+        if status != _lib.ST_OK:
             raise dense.CholeskyError("Cholesky decomposition was not successful: the GP system "
                                       "matrix is not positive definite")
         return float(out[0]), out[5:9].copy(), out
