@@ -99,6 +99,9 @@ SIGNATURES = {
                              P, S, P, P, P]),
 }
 
+# a launch per term, step, column or block
+LAUNCH_LOOPS = ("rvgp_cheb_series", "rvgp_batch_steps", "rvgp_syev", "rvgp_potrf", "rvgp_trsm")
+
 RVGP_EINVAL, RVGP_ERUNTIME, RVGP_ENOMEM, RVGP_EHIP = -1, -2, -3, -4
 ST_OK, ST_RANK_DEFICIENT, ST_SHORT_COMPONENT, ST_POOL_OVERFLOW, ST_NOT_SPD, ST_TIMEOUT = \
     0, 1, 2, 3, 4, 5
@@ -106,14 +109,18 @@ ST_OK, ST_RANK_DEFICIENT, ST_SHORT_COMPONENT, ST_POOL_OVERFLOW, ST_NOT_SPD, ST_T
 
 def load_symbols_only():
     """Load the library without touching the GPU (used by CPU tests)."""
-    # The interpreter's lock is kept over a call: an entry point launches and
-    # returns in microseconds and never waits for the GPU.  Giving the lock up at
-    # every launch made the two threads of a data object's spectra wake each other
-    # thousands of times (8000 nodes: 42.8 -> 35 ms, 20000: 42.9 -> 37 ms).
-    L = ctypes.PyDLL(LIB_PATH)
+    # The interpreter's lock is kept over a call of a few launches, which returns
+    # in microseconds: giving it up at every launch made the two threads of a data
+    # object's spectra wake each other thousands of times (8000 nodes: 42.8 -> 35
+    # ms, 20000: 42.9 -> 37 ms).  Entry points that launch in a loop give it up: they
+    # take as long as their launches do, and wait for the GPU where its queue is
+    # full (8000 nodes, 150 pairs, mixed: 35.8 ms with the lock kept over them too,
+    # 33.8 ms; 20000 nodes in R^32, 200 pairs: 54 and 50 ms).
+    L, unlocked = ctypes.PyDLL(LIB_PATH), ctypes.CDLL(LIB_PATH)
     for name, (res, args) in SIGNATURES.items():
-        fn = getattr(L, name)
+        fn = getattr(unlocked if name in LAUNCH_LOOPS else L, name)
         fn.restype, fn.argtypes = res, args
+        setattr(L, name, fn)
     return L
 
 
