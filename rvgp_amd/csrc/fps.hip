@@ -125,6 +125,10 @@ __global__ __launch_bounds__(kFpsThreads) void fps_kernel(
     int count = n_iter;
     for (int it = 1; it < n_iter; ++it) {
         ArgMax am = block_argmax(bv, bi, sv, si);
+        if (am.v < 0.0) {  // every distance is NaN: no point to select (am.i is none)
+            count = it;
+            break;
+        }
         if (threadIdx.x == 0) {
             perm[it] = am.i;
             lambdas[it] = am.v;
