@@ -15,9 +15,13 @@ namespace rvgp {
 // mode 2: v = T T^T v (in/out: (F, n, D))
 // G lanes per node, lane p its ambient coordinates p, p + G, ...: vectors and
 // frames are read and written in the order they are stored, and for D <= G a
-// node's frame stays in registers for all F fields; the sums over D meet by
-// shuffles.  (A thread per node and field read both 256 bytes apart: n =
+// node's frame stays in registers for all of its workgroup's fields (blockIdx.y,
+// blockIdx.y + gridDim.y, ...); the sums over D meet by shuffles.  (A thread per node and field read both 256 bytes apart: n =
 // 50,000, F = 16, D = 32, d = 3, 2.1 ms -> 0.17 (mode 0) and 0.10 ms (mode 1), bound by HBM.)
+// workgroups that fill the GPU: 2000 fields of 5000 nodes in R^3 take 249, 240 and
+// 223 us with 2048, 4096 and 16384, of 512 nodes 23, 23 and 29 us
+constexpr int kFrameGroups = 4096;
+
 template <int G>
 __global__ __launch_bounds__(256) void frame_kernel(int mode, int F, int n, int D, int d, int ldt,
                                                     const double* __restrict__ T,
@@ -34,7 +38,7 @@ __global__ __launch_bounds__(256) void frame_kernel(int mode, int F, int n, int 
         for (int q = 0; q < DM; ++q) t[q] = live && q < d && p < D ? Ti[(size_t)p * ldt + q] : 0.0;
     };
     if (once) frame_row(l);
-    for (int f = 0; f < F; ++f) {
+    for (int f = blockIdx.y; f < F; f += gridDim.y) {
         const size_t g = (size_t)f * n + (live ? i : 0);
         double c[DM];
         if (mode == 1) {
@@ -124,7 +128,10 @@ extern "C" int rvgp_frame_apply(int mode, int F, int n, int D, int d, const doub
     const size_t rows = (size_t)F * n;
     if (rows == 0) return RVGP_OK;
     const int G = D <= 4 ? 4 : D <= 8 ? 8 : D <= 16 ? 16 : D <= 32 ? 32 : 64;
-    const dim3 grid(cdiv((size_t)n * G, 256)), block(256);
+    // few nodes: the fields are split until the GPU is full (2000 fields, one
+    // workgroup for all of them: 64 nodes in R^3 1690 us, 8 us split)
+    const unsigned nodes = cdiv((size_t)n * G, 256), fill = cdiv(kFrameGroups, nodes);
+    const dim3 grid(nodes, (unsigned)F < fill ? (unsigned)F : fill), block(256);
     hipStream_t s = as_stream(stream);
 #define RVGP_FRAME(GG) \
     hipLaunchKernelGGL((frame_kernel<GG>), grid, block, 0, s, mode, F, n, D, d, ldt, T, in, out)
