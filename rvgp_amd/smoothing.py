@@ -60,7 +60,14 @@ class _Series:
         self.t0 = torch.zeros((X.shape[0], ld), **f64)
         self.t0[:, :r] = X if self.order is None else X[:, order]
         self.t1, self.out = torch.empty_like(self.t0), torch.empty_like(self.t0)
-        self.coef = torch.as_tensor(C, device=X.device)
+        if len(ts) == 1 and torch.cuda.is_current_stream_capturing():
+            # one time for all columns: numbers that a capture can hold, where a
+            # copy from the host cannot be captured
+            self.coef = torch.empty((J, ld), **f64)
+            for row, c in zip(self.coef, made[ts[0]]):
+                row.fill_(float(c))
+        else:
+            self.coef = torch.as_tensor(C, device=X.device)
         lengths = np.array([len(cs[c]) for c in order])
         self.active = np.ascontiguousarray((lengths[None, :] > np.arange(J)[:, None]).sum(1), np.int32)
         # T_1 = (2/ubs)(A - shift) X - X ; T_j = (4/ubs)(A - shift) T_{j-1} - 2 T_{j-1} - T_{j-2}

@@ -75,3 +75,28 @@ def test_frame_maps(D, d, n, F):
         _lib.call("rvgp_frame_apply", mode, F, n, D, d, _lib.ptr(Td), d + 1, _lib.ptr(xd), _lib.ptr(out),
                   _lib.stream())
         np.testing.assert_allclose(out.cpu().numpy(), ref, rtol=1e-12, atol=1e-12 * D * d)
+
+
+@pytest.mark.parametrize("columns", [1, 3, 16])
+def test_series_of_one_time_can_be_captured(columns):
+    import torch
+    from rvgp_amd import smoothing
+    from rvgp_amd.sparse import BSR
+    A, L = BSR.from_scipy(_laplacian(400, 2, 5), 2), BSR.from_scipy(_laplacian(400, 1, 6), 1)
+    X = torch.randn(800, columns, dtype=torch.float64, device="cuda")
+    c = torch.randn(400, 2, dtype=torch.float64, device="cuda")
+    ub = A.spectral_upper_bound()
+
+    def step():
+        return smoothing.expm_multiply(A, X, 0.7, ub=ub), smoothing.vector_diffusion_device(c, 0.7, A, L)
+
+    step()  # the operators' bounds, which a capture cannot compute
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = step()
+    for k in range(4):
+        X.normal_()
+        c.normal_()
+        g.replay()
+        for got, ref in zip(out, step()):
+            assert torch.equal(got, ref), k
