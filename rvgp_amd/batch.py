@@ -30,7 +30,10 @@ GAUSSIAN_VARIANCE_LOWER_BOUND = 1e-6
 # Fits of up to this many eigenvectors keep their factor in LDS, and one launch
 # runs many steps of them (kLdsTiles in batch.hip): a launch a step, replayed
 # from a graph, took 70 us at k = 120, a step of many in one launch 45 us.
-# Enough steps to lose the launch, few enough that a launch stays near 2 ms.
+# Enough steps to lose the launch, few enough that a launch stays near 2 ms.  The
+# other launch shapes are not tried for them: panels of 32 from memory take 1.2
+# to 4.5 times as long a step for 2 to 600 fits of k = 8 to 160 (256 fits of k =
+# 64: 45 us against 155).
 LDS_MAX_K = 160
 STEPS_PER_LAUNCH = 50
 
@@ -124,7 +127,9 @@ class BatchedGPR:
         if grid is None:
             grid = torch.cuda.get_device_properties(dev).multi_processor_count
         self.grid = int(grid)
-        if panel is None:
+        if panel is None and k <= LDS_MAX_K:
+            panel = (16, 512)
+        elif panel is None:
             panel = autotune.choose("batch_step", f"F{F},k{k},grid{self.grid}",
                                     ((16, 512), (16, 1024), (32, 512), (32, 1024)),
                                     lambda c: self._step(0, 0.0, panel=c))
@@ -230,7 +235,8 @@ def fit_batched(data, train_sets, vectors=None, epochs=200, lr=0.05, kernel=None
                 gram_precision="fp64", use_graph=True, timings=None):
     """Fit one GP per field of `vectors` (F, n, D) -- default data.vectors --
     each on its own node subset train_sets[f], all at once (Adam, device
-    resident, one graph-captured launch per step).  Hyperparameters start at
+    resident: many steps a launch up to LDS_MAX_K eigenvectors, else a launch a
+    step, captured in a graph unless use_graph is False).  Hyperparameters start at
     the Matern defaults of RVGP.fit (nu=3/2, kappa=5, sigma_f=1, main.py:30)
     and the given noise variance, or at theta0 ((4,) or (F, 4))."""
     import time

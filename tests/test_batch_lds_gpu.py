@@ -121,3 +121,17 @@ def test_many_steps_in_one_call_equal_single_calls(k):
     for other in got[1:]:
         for x, y in zip(got[0], other):
             np.testing.assert_array_equal(x, y)
+
+
+def test_launch_shapes_are_timed_only_where_they_differ():
+    """Up to LDS_MAX_K one kernel serves: nothing to time on a new problem shape."""
+    import torch
+    import rvgp_amd as RVGP
+    from rvgp_amd import autotune
+    from tests.util import torus
+    d = RVGP.create_data_object(torus(400, 2), n_neighbors=12, n_eigenpairs=20, verbose=False)
+    V = torch.randn(3, 400, 3, dtype=torch.float64, device="cuda")
+    sets = [np.arange(f, 200 + 7 * f) for f in range(3)]
+    gp = RVGP.fit_batched(d, sets, vectors=V, epochs=2)
+    assert (gp.panel, gp.threads) == (16, 512)
+    assert not [key for key in autotune.table() if key.startswith("batch_step|") and ",k20," in key]
