@@ -21,15 +21,28 @@ def _dev_f64(x):
 # a1  geometry.py:126-162
 # ---------------------------------------------------------------------------
 def _fps_blocked(n, D, n_iter):
-    """Whether the loop over spatial blocks (rvgp_fps_blocks) is the faster
-    one.  Its order and blocks cost ~0.2 ms (0.5 ms with principal axes), a
-    selection ~2 us (6 us for D = 32); the plain loop takes 2.8 us a selection
-    at n = 500, 15 us at n = 20,000 (9 us and 70 us for D = 32 at 500 and
-    5,000), and up to 4096 points of D <= 3 it runs in registers, faster than
-    the blocks (n = 4000: 5.2 against 5.7 ms for 3000 selections)."""
+    """Whether the loop over spatial blocks (rvgp_fps_blocks) is the faster one.
+
+    Up to D = 3 it is from where the plain loop leaves registers (n = 4097, 64
+    selections: 0.37 against 0.37 ms; 400: 1.1 against 2.1 ms; in registers n =
+    4000, 3000 selections: 5.7 against 5.2 ms).  For more dimensions what it
+    saves has to pay for the order and blocks, and beyond D = 6 for principal axes
+    (most of it where the points lie in fewer dimensions and eigenvalues
+    cluster).  The plain loop's time a selection is known; of it the blocks save
+    30 % (D <= 6) or 60 % at the least but for points that fill six dimensions
+    (n = 2000, 400 selections: 2.1 against 2.0 ms).  On either side of the line,
+    blocks against plain: D = 4, n = 5000, 64 selections 0.41 to 0.55 against
+    0.44, n = 20,000 0.56 to 0.82 against 1.2; D = 32, n = 2000, 64 selections 1.2
+    to 2.3 against 1.9, n = 5000 2.0 to 2.6 against 4.6; D = 64, 400 selections, n =
+    512 2.9 to 8.5 against 6.5, n = 2000 7.8 to 10.6 against 22.8 ms."""
     if D > 64 or n > 4096 * 64 or n_iter < 64:
         return False
-    return n > 4096 if D <= 3 else n >= 512
+    if D <= 3:
+        return n > 4096
+    plain = 2.5 + n * D * (2e-4 if D <= 8 else 4.3e-4)  # us a selection
+    if n < 512:
+        return False
+    return 0.3 * plain * n_iter >= 200 if D <= 6 else 0.6 * plain * n_iter >= 400 + 1.8 * D * D
 
 
 def furthest_point_sampling_device(x, N=None, spacing=0.1, start_idx=0):
