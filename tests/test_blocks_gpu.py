@@ -105,3 +105,44 @@ def test_manifold_graph_over_blocks_matches_the_oracle(n, D, k):
     rp, c = cpu.sym_csr(cpu.knn(x, k))
     np.testing.assert_array_equal(g.rowptr.cpu().numpy(), rp)
     np.testing.assert_array_equal(g.cols.cpu().numpy(), c)
+
+
+# more dimensions than box coordinates: points of a 3-torus in R^32, and clouds
+# that fill their space, where no block can be skipped
+@pytest.mark.parametrize("n,D,N,kind", [(1500, 32, 400, "torus"), (1500, 32, 400, "cloud"), (2000, 7, 400, "cloud"),
+                                        (700, 12, 400, "cloud"), (2100, 64, 400, "cloud")])
+def test_fps_over_blocks_by_principal_axes(n, D, N, kind):
+    from rvgp_amd import geometry
+    assert geometry._fps_blocked(n, D, N)
+    x = flat_torus3(n, 1) if kind == "torus" else np.random.default_rng(D).normal(size=(n, D))
+    p, lam = geometry.furthest_point_sampling(x, N=N)
+    p_ref, lam_ref = cpu.fps(x, N=N)
+    np.testing.assert_array_equal(p, p_ref)
+    np.testing.assert_array_equal(lam, lam_ref)
+
+
+def test_fps_of_the_most_points_that_blocks_take():
+    """Past 131,072 points a block's coordinates are not kept in LDS."""
+    from rvgp_amd import geometry
+    x = torus(140001, 3)
+    p, lam = geometry.furthest_point_sampling(x, N=70)
+    p_ref, lam_ref = cpu.fps(x, N=70)
+    np.testing.assert_array_equal(p, p_ref)
+    np.testing.assert_array_equal(lam, lam_ref)
+
+
+@pytest.mark.parametrize("n,D,k", [(12500, 10, 12), (12001, 32, 20)])
+def test_graph_of_points_whose_blocks_cannot_be_skipped(n, D, k):
+    """A cloud that fills its space: the order says so, and the plain scan runs."""
+    import torch
+    from rvgp_amd import geometry
+    from rvgp_amd.reorder import SpatialOrder
+    x = np.random.default_rng(n).normal(size=(n, D))
+    xd = torch.as_tensor(x, device="cuda")
+    order = SpatialOrder(xd)
+    top, prunes = order.prunes(order.blocks(transposed=False), xd.abs().max())
+    assert top == np.abs(x).max() and not prunes
+    g = geometry.manifold_graph(x, n_neighbors=k)
+    rp, c = cpu.sym_csr(cpu.knn(x, k))
+    np.testing.assert_array_equal(g.rowptr.cpu().numpy(), rp)
+    np.testing.assert_array_equal(g.cols.cpu().numpy(), c)
