@@ -68,9 +68,8 @@ constexpr int LDT = TB + 1;     // LDS tile row stride
 constexpr int kSpinLimit = 1 << 21;
 // L_qq^2 / A_qq below which explicit inverses lose more than a digit.  (At 1e-4
 // the NLML of 300 rows on half a circle, s2 = 1e-4, was off by 3e-5 unnoticed.)
-// Rows of nodes all over the manifold stay far above: such a step takes as long
-// as without the test (88 us at k = 200, 185 us at 500), a refined one 111 and
-// 229 us.
+// Rows of nodes all over the manifold stay far above: such a step takes 89 us at k
+// = 200 and 189 at 500, 87 and 182 without the test, a refined one 110 and 225.
 constexpr double kIll = 1e-2;
 
 // task numbering.  L column j: the diagonal task (which also produces
@@ -124,7 +123,7 @@ __host__ __device__ inline int lflag(const Layout& g, int i, int j) {
 }
 
 struct StepArgs {
-    int k, typ, ldg, do_adam, refine;
+    int k, typ, ldg, do_adam;
     double n_rows, M, lr, b1, b2, eps;
     const double* lam;
     const double* G;
@@ -420,6 +419,7 @@ __device__ __forceinline__ void correct_panel(dbl4& l, double* C, double* tmp, c
     tile_mma<true>(l, C, LDT, D, ldd, 1.0, qi, qj, lane);
 }
 
+template <bool REFINE>
 __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, double* lds) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int qi = wv >> 1, qj = wv & 1, T = g.T;
@@ -451,9 +451,10 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
             filter_terms(a.typ, a.lam[row], nu, kappa, r, dn, dk);
             add = s2 / floored(sf * a.n_rows * r / sr);
         }
-        if (row < a.k) diag = a.G[(size_t)row * a.ldg + row] + add;
+        if (REFINE && row < a.k) diag = a.G[(size_t)row * a.ldg + row] + add;
         dadd[tid] = add;
         adiag[tid] = diag;
+        if (tid == 0) adiag[TB] = 0.0;
     }
     __syncthreads();
     // C(j,j) and, below it, C(j+1,j): every update but C(j+1,j)'s last one
@@ -483,8 +484,9 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
     double* Ws = Ds + TB * LDT;  // 16 x 17 scratch
     // the first n pivots kept too little of A's diagonal
     auto ill = [&](int n) {
+        if (!REFINE) return false;
         const double d = Ls[(lane & 31) * (LDT + 1)];
-        return a.refine && __any(lane < n && d * d < kIll * adiag[lane & 31]);
+        return __any(lane < n && d * d < kIll * adiag[lane & 31]) != 0;
     };
     if (wv == 0) {
         // upper-right 16 x 16 blocks of L and D are zero; the rest is written
@@ -520,7 +522,7 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
         bad = (int)wave_max((double)bad);
         if (bad && lane == 0) atomicOr(ctl + 2, 1);
         const bool lost = ill(32);
-        if (lane == 0) {
+        if (REFINE && lane == 0) {
             if (lost) atomicOr(ctl + 3, 1);
             adiag[TB] = lost;
             a.ws[g.oP + 8 * (size_t)j + 7] = lost;  // for the panel tasks; free until column j's sums
@@ -545,7 +547,7 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
         // L(j+1,j) = C(j+1,j) D(j)^T
         dbl4 l1 = dbl4{0, 0, 0, 0};
         tile_mma<true>(l1, C1, LDT, Ds, LDT, 1.0, qi, qj, lane);
-        if (adiag[TB] != 0.0) correct_panel(l1, C1, Cs, Ls, LDT, Ds, LDT, qi, qj, lane);
+        if (REFINE && adiag[TB] != 0.0) correct_panel(l1, C1, Cs, Ls, LDT, Ds, LDT, qi, qj, lane);
         quad_store(l1, Lt + (size_t)tix(j + 1, j) * TT, TB, qi, qj, lane);
     }
     {
@@ -560,6 +562,7 @@ __device__ void task_diag(const StepArgs& a, const Layout& g, int j, int epoch, 
     publish(sync + g.fD + j, epoch);
 }
 
+template <bool REFINE>
 __device__ void task_offdiag(const StepArgs& a, const Layout& g, int i, int j, int epoch,
                              double* lds) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -581,7 +584,7 @@ __device__ void task_offdiag(const StepArgs& a, const Layout& g, int i, int j, i
     dbl4 l = dbl4{0, 0, 0, 0};
     const double* D = Xt + (size_t)tix(j, j) * TT;
     tile_mma<true>(l, Cs, LDT, D, TB, 1.0, qi, qj, lane);  // C D(j)^T
-    if (a.refine && a.ws[g.oP + 8 * (size_t)j + 7] != 0.0)
+    if (REFINE && a.ws[g.oP + 8 * (size_t)j + 7] != 0.0)
         correct_panel(l, Cs, Cs + TB * LDT, Lt + (size_t)tix(j, j) * TT, TB, D, TB, qi, qj, lane);
     quad_store(l, Lt + (size_t)tix(i, j) * TT, TB, qi, qj, lane);
     publish(sync + lflag(g, i, j), epoch);
@@ -736,6 +739,7 @@ __device__ void task_row(const StepArgs& a, const Layout& g, int i, int epoch, b
 // where y^T y - b^T w of the other form cancels to s2 times its terms.  Both
 // hold for any c; P[7] is the part of y in directions of Phi that the split
 // left in e.
+template <bool REFINE>
 __device__ void task_col(const StepArgs& a, const Layout& g, int j, int epoch, double* lds, bool second) {
     const int tid = threadIdx.x, T = g.T, k = a.k;
     int* sync = a.sync;
@@ -745,8 +749,10 @@ __device__ void task_col(const StepArgs& a, const Layout& g, int j, int epoch, d
     const double* tv = a.ws + (second ? g.oA : g.oT);
     const int c = tid & 31, q = tid >> 5;
     double sw = 0.0, sa = 0.0;
+    // row i has seen every X(i, .); the corrections come all at about the same time
+    if (second) wait_all([&](int i) { return sync + g.fR + j + i; }, T - j, epoch + 2, ctl);
     for (int i = j; i < T; ++i) {
-        wait_for(sync + g.fR + i, second ? epoch + 2 : epoch, ctl);  // row i has seen every X(i, .)
+        if (!second) wait_for(sync + g.fR + i, epoch, ctl);
         const double* X = Xt + (size_t)tix(i, j) * TT;
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
@@ -756,7 +762,7 @@ __device__ void task_col(const StepArgs& a, const Layout& g, int j, int epoch, d
             sa += x * x;
         }
     }
-    const bool more = a.refine && ld_flag(ctl + 3) != 0;  // the last row is there (refining())
+    const bool more = REFINE && ld_flag(ctl + 3) != 0;  // the last row is there (refining())
     double* pw = lds;            // 8 x 32
     double* pa = lds + 8 * TB;   // 8 x 32
     pw[q * TB + c] = sw;
@@ -803,20 +809,21 @@ __device__ void task_col(const StepArgs& a, const Layout& g, int j, int epoch, d
 #pragma unroll
             for (int m = 0; m < 8; ++m) a.ws[g.oP + 8 * (size_t)j + m] = v[m];
     }
-    publish(sync + g.fC + j, a.refine && second == more ? epoch + 1 : epoch);  // the sums are there
+    publish(sync + g.fC + j, REFINE && second == more ? epoch + 1 : epoch);  // the sums are there
 }
 
 // NLML and adjoint (gp.hip's weight-space finish, one right-hand side, with
 // w^T G w = b^T w - s2 sum_j w_j^2 / S_j since A w = b) from the column
 // partials, summed in tile order; then Adam.
+template <bool REFINE>
 __device__ void task_final(const StepArgs& a, const Layout& g, int epoch) {
     const int tid = threadIdx.x, T = g.T, k = a.k;
     int* sync = a.sync;
     int* ctl = sync + g.ctl;
     // the column tasks all finish after the last row: wait for them (and the
     // filter) at once
-    wait_all([&](int j) { return j < T ? sync + g.fC + j : sync + g.fF; }, a.refine ? T : T + 1,
-             a.refine ? epoch + 1 : epoch, ctl);
+    wait_all([&](int j) { return j < T ? sync + g.fC + j : sync + g.fF; }, REFINE ? T : T + 1,
+             REFINE ? epoch + 1 : epoch, ctl);
     if (tid < 4) {
         const int p = tid;
         double P[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -864,10 +871,11 @@ __device__ void task_final(const StepArgs& a, const Layout& g, int epoch) {
         st_flag(ctl + 1, 0);
         st_flag(ctl + 2, 0);
         st_flag(ctl + 3, 0);
-        st_flag(ctl, a.refine ? epoch + 2 : epoch);  // the next launch runs one more
+        st_flag(ctl, REFINE ? epoch + 2 : epoch);  // the next launch runs one more
     }
 }
 
+template <bool REFINE>
 __global__ __launch_bounds__(NTH) void ws_step_kernel(StepArgs a) {
     __shared__ double lds[4 * TB * LDT + 16 * 17 + 72];
     __shared__ int s_epoch;
@@ -884,8 +892,8 @@ __global__ __launch_bounds__(NTH) void ws_step_kernel(StepArgs a) {
         int j = 0;
         while (j + 1 < T && lbase(T, j + 1) <= b) ++j;
         const int off = b - lbase(T, j);
-        if (off == 0) task_diag(a, g, j, epoch, lds);
-        else task_offdiag(a, g, j + 1 + off, j, epoch, lds);
+        if (off == 0) task_diag<REFINE>(a, g, j, epoch, lds);
+        else task_offdiag<REFINE>(a, g, j + 1 + off, j, epoch, lds);
         return;
     }
     b -= g.nL;
@@ -901,12 +909,12 @@ __global__ __launch_bounds__(NTH) void ws_step_kernel(StepArgs a) {
     b -= 1;
     if (b < T) { task_row(a, g, b, epoch, false); return; }
     b -= T;
-    if (b < T) { task_col(a, g, b, epoch, lds, false); return; }
+    if (b < T) { task_col<REFINE>(a, g, b, epoch, lds, false); return; }
     b -= T;
-    if (a.refine && b < T) { task_residual(a, g, b, epoch); return; }
-    if (a.refine && b < 2 * T) { task_row(a, g, b - T, epoch, true); return; }
-    if (a.refine && b < 3 * T) { task_col(a, g, b - 2 * T, epoch, lds, true); return; }
-    task_final(a, g, epoch);
+    if (REFINE && b < T) { task_residual(a, g, b, epoch); return; }
+    if (REFINE && b < 2 * T) { task_row(a, g, b - T, epoch, true); return; }
+    if (REFINE && b < 3 * T) { task_col<REFINE>(a, g, b - 2 * T, epoch, lds, true); return; }
+    task_final<REFINE>(a, g, epoch);
 }
 
 }  // namespace
@@ -944,8 +952,9 @@ static int ws_step(const double* c, const double* ge, int k, int typ, const doub
     a.ldg = ldg;
     a.do_adam = do_adam;
     // a host optimiser's evaluations and the split form; an Adam step of the
-    // weight form, whose y^T y - b^T w loses as much, does without
-    a.refine = c != nullptr || !do_adam;
+    // weight form, whose y^T y - b^T w loses as much, does without (a kernel of
+    // its own: the unused branches cost 2 us of 87)
+    const bool refine = c != nullptr || !do_adam;
     a.c = c;
     a.g = ge;
     a.n_rows = n_rows;
@@ -968,8 +977,8 @@ static int ws_step(const double* c, const double* ge, int k, int typ, const doub
     a.sync = sync;
     a.out = out;
     a.status = status;
-    hipLaunchKernelGGL(ws_step_kernel, dim3(g.nblocks + (a.refine ? 3 * g.T : 0)), dim3(NTH), 0,
-                       as_stream(stream), a);
+    hipLaunchKernelGGL(refine ? ws_step_kernel<true> : ws_step_kernel<false>,
+                       dim3(g.nblocks + (refine ? 3 * g.T : 0)), dim3(NTH), 0, as_stream(stream), a);
     RVGP_LAUNCH_CHECK();
     return RVGP_OK;
 }

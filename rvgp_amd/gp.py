@@ -303,7 +303,7 @@ class GPREngine:
     def evaluate(self):
         """Enqueue NLML + gradient; results in self.out (device):
         [nlml, d/d(nu, kappa, sigma_f, s2), d/du(...)].  One launch where the
-        single-launch step serves the fit (k = 500: 185 against 356 us)."""
+        single-launch step serves the fit (k = 500: 189 against 356 us, 225 us where it refines)."""
         return self._ws_step(0) if self.fused() else self._evaluate_state()
 
     def _evaluate_state(self):
