@@ -46,6 +46,9 @@ class _Series:
     columns ordered by the length of their series, the row stride even."""
 
     def __init__(self, A, X, ts, ub, shift):
+        # the kernel reads X's rows by A's columns
+        assert X.dim() == 2 and X.shape[0] == A.shape[0], (X.shape, A.shape)
+        _lib.ptr(X)
         r = X.shape[1]
         ubs = ub - shift
         made = {t: cheb_coeffs(t, ubs) for t in set(ts)}
@@ -71,8 +74,8 @@ class _Series:
         lengths = np.array([len(cs[c]) for c in order])
         self.active = np.ascontiguousarray((lengths[None, :] > np.arange(J)[:, None]).sum(1), np.int32)
         # T_1 = (2/ubs)(A - shift) X - X ; T_j = (4/ubs)(A - shift) T_{j-1} - 2 T_{j-1} - T_{j-2}
-        self.op = _lib.Series(A.nb, A.b, *(t.data_ptr() for t in (A.rowptr, A.cols, A.vals64, self.t0,
-                                                                  self.t1, self.out, self.coef)),
+        self.op = _lib.Series(A.nb, A.b, *map(_lib.ptr, (A.rowptr, A.cols, A.vals64, self.t0, self.t1,
+                                                        self.out, self.coef)),
                               ld, J, self.active.ctypes.data, 4.0 / ubs, -2.0 - 4.0 * shift / ubs)
 
     def result(self):
@@ -113,6 +116,8 @@ def expm_multiply(A: BSR, X, t, ub=None, shift=0.0):
     shift = max(float(shift), 0.0)
     X2 = X.reshape(-1, 1) if X.dim() == 1 else X
     ts = _times(t, X2.shape[1])
+    if X2.shape[1] == 0:
+        raise ValueError("expm_multiply: X has no columns")
     if X2.dtype != torch.float64:
         return _expm_spmm(A, X2, ts, ub, shift).reshape(X.shape)
     parts = []
@@ -171,6 +176,7 @@ def vector_diffusion_device(c, t, Lc: BSR, L: BSR, lc_min=0.0, perm=None):
     c and the result are not."""
     batched = c.dim() == 3
     C = c if batched else c.unsqueeze(0)
+    assert (C.shape[1] * C.shape[2], C.shape[1]) == (Lc.shape[0], L.shape[0]), (c.shape, Lc.shape, L.shape)
     if perm is not None:
         C = C.index_select(1, perm)
     F, n, d = C.shape
