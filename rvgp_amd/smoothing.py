@@ -134,6 +134,16 @@ def _expm_spmm(A, X2, ts, ub, shift):
     """The series by block SpMMs, for blocks of other types than FP64."""
     ubs = ub - shift
     cs = [cheb_coeffs(tc, ubs) for tc in ts]
+    if len(ts) == 1 and shift == 0.0:
+        # one coefficient a term: the product adds it to the sum
+        c = cs[0]
+        out = X2 * float(c[0])
+        T1 = spmm(A, X2, alpha=2.0 / ub, beta=-1.0, acc=out, delta=float(c[1]))
+        prev, cur = X2.clone(), T1
+        for j in range(2, len(c)):
+            spmm(A, cur, Y=prev, alpha=4.0 / ub, beta=-2.0, Z=prev, gamma=-1.0, acc=out, delta=float(c[j]))
+            prev, cur = cur, prev
+        return out
     C = np.zeros((max(len(c) for c in cs), X2.shape[1]))
     for col in range(X2.shape[1]):
         c = cs[col if len(ts) > 1 else 0]

@@ -100,3 +100,25 @@ def test_series_of_one_time_can_be_captured(columns):
         g.replay()
         for got, ref in zip(out, step()):
             assert torch.equal(got, ref), k
+
+
+def test_series_in_single_precision_can_be_captured():
+    """Blocks of other types than FP64 take the block SpMMs, one launch a term for
+    one diffusion time."""
+    import torch
+    from rvgp_amd.smoothing import expm_multiply
+    from rvgp_amd.sparse import BSR
+    A = _laplacian(300, 3, 9)
+    B = BSR.from_scipy(A, 3)
+    x = np.random.default_rng(0).normal(size=(900, 4))
+    X = torch.as_tensor(x, dtype=torch.float32, device="cuda")
+    ub = B.spectral_upper_bound()
+    # a few hundred terms of FP32 rounding on values of size 1
+    np.testing.assert_allclose(expm_multiply(B, X, 0.7, ub=ub).cpu().numpy(), _heat(A, x, [0.7] * 4), atol=1e-4)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = expm_multiply(B, X, 0.7, ub=ub)
+    for _ in range(3):
+        X.normal_()
+        g.replay()
+        assert torch.equal(out, expm_multiply(B, X, 0.7, ub=ub))
