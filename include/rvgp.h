@@ -223,7 +223,7 @@ int rvgp_frame_apply(int mode, int F, int n, int D, int d, const double* T, int 
 /* One Chebyshev series on a block-CSR operator (block size b = 1, 2, 3; FP64):
  * out = sum_{j < terms} C_j o T_j with T_0 in t0, T_1 = (a A + shift) T_0 / 2,
  * T_j = (a A + shift) T_{j-1} - T_{j-2}; t0 and t1 are overwritten.  Blocks are
- * nb*b rows of ld <= 64 doubles (even, 16-byte aligned, unused columns zero);
+ * nb*b rows of ld doubles (even, 16-byte aligned, unused columns zero);
  * coef (terms, ld) on the device, a coefficient per term and column; active[j]
  * (HOST, non-increasing): the columns with coefficients from term j on. */
 typedef struct {

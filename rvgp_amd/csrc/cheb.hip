@@ -8,12 +8,14 @@
 // of columns whose series has ended are not formed: columns come ordered by
 // the length of their series, and a term runs on the leading ones.
 //
-// Mapping: V lanes hold a row's columns (16-byte pairs), E lanes split its
-// stored blocks, so that a wave works on 64 / (V E) block rows whatever the
+// Mapping: V lanes hold a row's columns (16-byte pairs; past 64 columns in groups
+// of 64), E lanes split its stored blocks, so that a wave works on 64 / (V E) block rows whatever the
 // width -- one wave per row left 56 of 64 lanes idle at 16 columns.  n = 50,000,
 // b = 3, 16 columns: 122 + 8 (sum) -> 83 us a term, 57 us where the rows are numbered along a
 // space-filling curve; b = 1, 32 columns: 46 + 8 -> 42 and 25 us.
 // Bound by the gathers through L1 and L2.
+// All groups of columns share a term's launch: 100 fields on 600 nodes of a 3-torus
+// 12.8 ms a smoothing (t = 60) in blocks of 64 columns, 9.3 ms by SpMMs, 6.8 ms so.
 // Small operators are bound by the launches: the two series of a vector
 // diffusion (connection and scalar Laplacian) then share theirs.
 #include "common.h"
@@ -40,6 +42,7 @@ struct Series {
 };
 
 constexpr int kThreads = 256;
+constexpr int kColumns = 64;  // of a workgroup; more of them are gridDim.y
 
 template <int B, int V, int E>
 __device__ __forceinline__ void term_rows(const Series& s, int wg, int wgs) {
@@ -49,7 +52,7 @@ __device__ __forceinline__ void term_rows(const Series& s, int wg, int wgs) {
     const int lw = (wg & 7) * per + (wg >> 3);
     const int row = lw * ROWS + (int)threadIdx.x / G;
     const int l = threadIdx.x % G;
-    const int v = l % V, ed = l / V, c = 2 * v;
+    const int v = l % V, ed = l / V, c = 2 * v + kColumns * blockIdx.y;
     const bool on = row < s.nb && c < s.act;
     dbl2 y[B];
 #pragma unroll
@@ -117,7 +120,7 @@ int grid_of(int nb) { return 8 * (int)cdiv(cdiv(nb, rows_per_wg<V, E>()), 8); }
 
 template <int V, int E>
 void launch_term(const Series& s, int b, hipStream_t st) {
-    const dim3 g(grid_of<V, E>(s.nb)), t(kThreads);
+    const dim3 g(grid_of<V, E>(s.nb), cdiv(s.act, kColumns)), t(kThreads);
     if (b == 1) hipLaunchKernelGGL((term_kernel<1, V, E>), g, t, 0, st, s);
     else if (b == 2) hipLaunchKernelGGL((term_kernel<2, V, E>), g, t, 0, st, s);
     else hipLaunchKernelGGL((term_kernel<3, V, E>), g, t, 0, st, s);
@@ -135,8 +138,8 @@ extern "C" int rvgp_cheb_series(int nops, const rvgp_series* ops, void* stream) 
         const rvgp_series& p = ops[o];
         RVGP_CHECK_ARG(p.nb >= 1 && p.b >= 1 && p.b <= 3, "rvgp_cheb_series: block size must be 1, 2 or 3");
         RVGP_CHECK_ARG(p.terms >= 2 && p.active != nullptr, "rvgp_cheb_series: need at least two terms");
-        RVGP_CHECK_ARG(p.ld >= 2 && p.ld % 2 == 0 && p.ld <= 64,
-                       "rvgp_cheb_series: the row stride must be even and <= 64");
+        RVGP_CHECK_ARG(p.ld >= 2 && p.ld % 2 == 0 && p.ld <= 65535 * kColumns,
+                       "rvgp_cheb_series: the row stride must be even and at most %d", 65535 * kColumns);
         RVGP_CHECK_ARG((((uintptr_t)p.t0 | (uintptr_t)p.t1 | (uintptr_t)p.out | (uintptr_t)p.coef) % 16) == 0 &&
                            p.t0 != p.t1 && p.t0 != p.out && p.t1 != p.out,
                        "rvgp_cheb_series: buffers must be distinct and 16-byte aligned");

@@ -38,11 +38,8 @@ def cheb_coeffs(t, ub, rtol=1e-17, max_terms=200000):
     return c[:max(J, 2)]
 
 
-SERIES_COLUMNS = 64  # most columns of one rvgp_cheb_series block
-
-
 class _Series:
-    """exp(-t (A - shift)) X for an FP64 X (rows, r <= 64) as an rvgp_series:
+    """exp(-t (A - shift)) X for an FP64 X (rows, r) as an rvgp_series:
     columns ordered by the length of their series, the row stride even."""
 
     def __init__(self, A, X, ts, ub, shift):
@@ -120,14 +117,9 @@ def expm_multiply(A: BSR, X, t, ub=None, shift=0.0):
         raise ValueError("expm_multiply: X has no columns")
     if X2.dtype != torch.float64:
         return _expm_spmm(A, X2, ts, ub, shift).reshape(X.shape)
-    parts = []
-    for c0 in range(0, X2.shape[1], SERIES_COLUMNS):
-        c1 = min(c0 + SERIES_COLUMNS, X2.shape[1])
-        s = _Series(A, X2[:, c0:c1], ts[c0:c1] if len(ts) > 1 else ts, ub, shift)
-        _run_series(s)
-        parts.append(s.result())
-    out = parts[0] if len(parts) == 1 else torch.cat(parts, 1)
-    return out.reshape(X.shape)
+    s = _Series(A, X2, ts, ub, shift)
+    _run_series(s)
+    return s.result().reshape(X.shape)
 
 
 def _expm_spmm(A, X2, ts, ub, shift):

@@ -37,3 +37,16 @@ def test_fields_of_other_nodes(n, d, perm):
 def test_no_columns():
     with pytest.raises(ValueError):
         expm_multiply(_operator(8, 1), torch.ones(8, 0, dtype=torch.float64), 0.5, ub=1.0)
+
+
+def test_the_library_takes_any_even_row_stride():
+    """Refused for its buffers alone (16-byte alignment), not for more than 64
+    columns: all columns of a series share a launch a term."""
+    import ctypes
+    from rvgp_amd import _lib
+    L = _lib.load_symbols_only()
+    active = (ctypes.c_int * 2)(130, 130)
+    for ld, word in ((130, b"aligned"), (131, b"even")):
+        op = _lib.Series(1, 1, 16, 16, 16, 8, 32, 48, 64, ld, 2, ctypes.addressof(active), 1.0, 0.0)
+        assert L.rvgp_cheb_series(1, ctypes.byref(op), None) == _lib.RVGP_EINVAL
+        assert word in L.rvgp_last_error()
