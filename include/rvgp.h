@@ -400,6 +400,18 @@ size_t rvgp_dot_ws_bytes(size_t n);
 int rvgp_dot(size_t n, const double* x, const double* y, double* out, void* ws, size_t ws_bytes,
              void* stream);
 
+/* The function-space form on the k x k system, from a split y = Phi c + e of the
+ * observations (k x nrhs arrays, row-major; ge = Phi^T e, ee = |e|^2) and w = A^-1
+ * Phi^T y: p = w / S = Phi^T K_y^-1 y, ya = y^T K_y^-1 y, aa = |K_y^-1 y|^2, for
+ * rvgp_fs_finish.  rvgp_coef_residual: r = b - s2 w / S, which less G w is the
+ * residual of A w = b. */
+size_t rvgp_coef_terms_ws_bytes(int k, int nrhs);
+int rvgp_coef_terms(int k, int nrhs, const double* c, const double* ge, const double* ee, const double* w,
+                    const double* S, const double* s2, double* p, double* ya, double* aa, void* ws,
+                    size_t ws_bytes, void* stream);
+int rvgp_coef_residual(int k, int nrhs, const double* b, const double* w, const double* S,
+                       const double* s2, double* r, void* stream);
+
 /* Determinant-lemma terms for the mixed-precision function-space form, from
  * the FP64 factor LA of A = s2 S^-1 + Phi^T Phi and diag(A^-1):
  * q_j = phi_j^T K_y^-1 phi_j and logdet_half = log det(K_y) / 2. */

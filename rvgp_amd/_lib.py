@@ -76,6 +76,9 @@ SIGNATURES = {
     "rvgp_fs_finish": (I, [I, D, I, P, P, P, P, P, P, P, P, P, P, P, P]),
     "rvgp_dot_ws_bytes": (S, [S]),
     "rvgp_dot": (I, [S, P, P, P, P, S, P]),
+    "rvgp_coef_terms_ws_bytes": (S, [I, I]),
+    "rvgp_coef_terms": (I, [I, I, P, P, P, P, P, P, P, P, P, P, S, P]),
+    "rvgp_coef_residual": (I, [I, I, P, P, P, P, P, P]),
     "rvgp_lemma_terms": (I, [I, D, P, P, P, P, I, P, P, P]),
     "rvgp_gp_params": (I, [P, P, P, P, P]),
     "rvgp_adam_step": (I, [P, P, P, P, P, P, D, D, D, D, P]),

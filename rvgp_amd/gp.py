@@ -88,7 +88,7 @@ FUSED_STEP_MAX_K = 2048  # RVGP_WS_STEP_MAX_K
 # Its flops are ~(k / M)^3 of the M x M factorisation's; below 2 k rows
 # Phi^T Phi is singular for the tangent fields' frames (rank m d < M).
 # M = 4731, k = 200: an evaluation 10.0 -> 0.09 ms (0.11 ms where Phi^T Phi is
-# close to singular and the step refines), building the engine 0.97 ms.
+# close to singular and the step refines), building the engine 0.54 ms.
 # Its error against 80-bit arithmetic, in brackets the M x M form's, on Fourier
 # columns (M = 300, k = 40) with noise 0.05, s2 = 0.1 ... 2e-6.  Nodes all over the
 # circle: NLML 6e-14 ... 9e-11 (3e-11 ... 4e-3), gradient <= 3e-15 of its largest
@@ -101,6 +101,7 @@ COEF_MIN_ROWS = 2
 # enough that little is left in e, large enough that c stays small in
 # directions where Phi^T Phi is rounding (1e-12: rounding of Phi c up to 3e-4 in
 # the NLML at s2 = 1e-6, 1e-6: 8e-4 from what is left; 1e-9: the least of both).
+# A second pass against the rows takes out no more than g accounts for already.
 SPLIT_RIDGE = 1e-9
 
 
@@ -180,7 +181,11 @@ class GPREngine:
                 self.ones = torch.ones(self.R, **f64)
                 self._cs_ws = torch.empty(
                     _lib.lib().rvgp_colsumsq_ws_bytes(self.M, self.R + self.k) // 8 + 1, **f64)
-            if not self.coef:
+            if self.coef:
+                self.p = torch.empty((self.k, self.R), **f64)
+                self._terms_ws = torch.empty(
+                    _lib.lib().rvgp_coef_terms_ws_bytes(self.k, self.R) // 8, **f64)
+            else:
                 self.a = torch.empty((self.M, self.R), **f64)
             self.q = torch.empty(self.k, **f64) if self.normal else self.colsq[self.R:]
             self.logdet = torch.empty(1, **f64)
@@ -216,25 +221,20 @@ class GPREngine:
 
     def _split_rows(self):
         """y = Phi c + e: c (k, R), |e|^2 and g = Phi^T e (k, R), by the Cholesky
-        factor of G with a ridge, two passes against the rows.  Duplicated
-        features, fewer tangent rows than features and nodes on a part of the
-        manifold leave G singular: the ridge makes it solvable, and what it
-        leaves in e of directions that the rows hold, g accounts for.  False
-        when G is not positive definite even so."""
+        factor of G with a ridge.  Duplicated features, fewer tangent rows than
+        features and nodes on a part of the manifold leave G singular: the ridge
+        makes it solvable, and what it leaves in e of directions that the rows
+        hold, g accounts for.  False when G is not positive definite even so."""
         L = self.G + (SPLIT_RIDGE * torch.diagonal(self.G).max()) * torch.eye(
             self.k, dtype=torch.float64, device=self.dev)
         _, st = dense.potrf(L, check=False)
         if int(st.item()) != 0:
             return False
-        c, g = torch.zeros_like(self.b), self.b
-        for _ in range(2):
-            r = g.clone()
-            dense.trsm(L, r)
-            dense.trsm(L, r, trans=True)
-            c = c + r
-            e = (self.y - dense.gemm(self.Phi, c)).contiguous()
-            g = dense.gemm(self.Phi, e, transA=True)
-        self.c, self.g = c.contiguous(), g
+        self.c = self.b.clone()
+        dense.trsm(L, self.c)
+        dense.trsm(L, self.c, trans=True)
+        e = (self.y - dense.gemm(self.Phi, self.c)).contiguous()
+        self.g = dense.gemm(self.Phi, e, transA=True)
         self.ee = torch.empty(1, dtype=torch.float64, device=self.dev)
         self._dot(e, e, self.ee)
         return True
@@ -325,9 +325,10 @@ class GPREngine:
             dense.gemm(self.Linv, t, self.w, transA=True)
             if self.coef:
                 # one refinement: L^-1 is good to cond(L), a solve with L to less
-                r = self.b - self.s2 * (self.w / self.S.reshape(-1, 1))
-                dense.gemm(self.G, self.w, r, alpha=-1.0, beta=1.0)
-                dense.gemm(self.Linv, dense.gemm(self.Linv, r), self.w, transA=True, beta=1.0)
+                _lib.call("rvgp_coef_residual", self.k, self.R, _lib.ptr(self.b), _lib.ptr(self.w),
+                          _lib.ptr(self.S), _lib.ptr(self.s2), _lib.ptr(self.p), s)
+                dense.gemm(self.G, self.w, self.p, alpha=-1.0, beta=1.0)
+                dense.gemm(self.Linv, dense.gemm(self.Linv, self.p), self.w, transA=True, beta=1.0)
         if self.form == "weight":
             Gw = dense.gemm(self.G, self.w)
             _lib.call("rvgp_ws_finish", self.k, float(self.M), self.R, _lib.ptr(self.A), self.k,
@@ -336,11 +337,11 @@ class GPREngine:
                       _lib.ptr(self.u), _lib.ptr(self.gS), _lib.ptr(self.out), s)
             return self.out
         if self.coef:
-            p = (self.w / self.S.reshape(-1, 1)).contiguous()  # Phi^T K_y^-1 y
-            d = (self.c - self.w).contiguous()
-            t = (self._dot(self.g, d, torch.empty_like(self.ee)) + self.ee) / self.s2
-            self._dot(self.c, p, self.ya).add_(t)
-            self._dot(p, d, self.aa).add_(t).div_(self.s2)
+            p = self.p  # Phi^T K_y^-1 y
+            _lib.call("rvgp_coef_terms", self.k, self.R, _lib.ptr(self.c), _lib.ptr(self.g),
+                      _lib.ptr(self.ee), _lib.ptr(self.w), _lib.ptr(self.S), _lib.ptr(self.s2),
+                      _lib.ptr(p), _lib.ptr(self.ya), _lib.ptr(self.aa), _lib.ptr(self._terms_ws),
+                      self._terms_ws.numel() * 8, s)
         elif self.precision == "mixed":
             # alpha = K_y^-1 y = (y - Phi w) / s2 (Woodbury; w = A^-1 Phi^T y
             # above), then two refinement sweeps against the FP64 K_y

@@ -129,9 +129,38 @@ def test_nodes_on_a_part_of_the_manifold(M, k, part, R, noise, s2):
     assert e.coef
     nlml, _, out = e.nlml_grad_u(e.u.cpu().numpy())
     ref, grad, S = _extended(Phi, y, lam, th, 500.0)
-    # rounding of Phi c, where |c| <= |y| / sqrt(ridge G), and of G, against s2; two
-    # passes of two products
+    # rounding of Phi c, where |c| <= |y| / sqrt(ridge G), and of G, against s2, in
+    # each of four products
     off = 4 * np.finfo(float).eps * ((y * y).sum() / np.sqrt(1e-9) + R * (Phi * Phi).sum(0) @ S) / s2
     assert abs(nlml - ref) <= off + 1e-9 * abs(ref)
     np.testing.assert_allclose(out[1:4], grad[:3], rtol=1e-7, atol=10 * off)
     np.testing.assert_allclose(out[4], grad[3], rtol=1e-9, atol=off / s2)
+
+
+# one and several slices of 2048 entries, remainders, the most slices
+@pytest.mark.parametrize("k,R", [(1, 1), (3, 7), (33, 64), (64, 32), (150, 2000), (2048, 1100)])
+def test_terms_of_the_split_form(k, R):
+    import torch
+    from rvgp_amd import _lib
+    rng = np.random.default_rng(k + R)
+    c, g, w, b = (rng.normal(size=(k, R)) for _ in range(4))
+    S, ee, s2 = np.exp(rng.normal(size=k)), np.array([3.7]), np.array([0.02])
+    S[k // 2], w[k // 2] = 1e-280, 1e-281 * w[k // 2]  # a filter value at its floor
+    dev = {n: torch.as_tensor(v, device="cuda") for n, v in dict(c=c, g=g, w=w, b=b, S=S, ee=ee, s2=s2).items()}
+    size = _lib.lib().rvgp_coef_terms_ws_bytes(k, R)
+    p, ws = torch.empty(k, R, dtype=torch.float64, device="cuda"), torch.empty(size // 8, dtype=torch.float64, device="cuda")
+    ya, aa = torch.empty(1, dtype=torch.float64, device="cuda"), torch.empty(1, dtype=torch.float64, device="cuda")
+    r = torch.empty_like(p)
+    _lib.call("rvgp_coef_terms", k, R, *[_lib.ptr(dev[n]) for n in ("c", "g", "ee", "w", "S", "s2")], _lib.ptr(p),
+              _lib.ptr(ya), _lib.ptr(aa), _lib.ptr(ws), size, _lib.stream())
+    _lib.call("rvgp_coef_residual", k, R, *[_lib.ptr(dev[n]) for n in ("b", "w", "S", "s2")], _lib.ptr(r), _lib.stream())
+    X = np.longdouble
+    pr = w / S[:, None]
+    np.testing.assert_array_equal(p.cpu().numpy(), pr)
+    np.testing.assert_allclose(r.cpu().numpy(), b - s2 * pr, rtol=0, atol=4e-16 * np.abs(b).max())
+    d = c.astype(X) - w
+    t = (X(3.7) + (g * d).sum()) / X(0.02)
+    cp, pd = (c * pr.astype(X)).sum(), (pr * d).sum()
+    # sums of k R products of numbers of size 1
+    off = 1e-15 * np.sqrt(k * R) * (1 + np.abs(pr).max()) * 10
+    assert abs(ya.item() - float(cp + t)) <= off * 60 and abs(aa.item() - float((pd + t) / X(0.02))) <= off * 60 * 60
