@@ -210,8 +210,8 @@ __global__ __launch_bounds__(FT) void dot_reduce_kernel(int parts, const double*
 // The split form's products over k x R entries, y = Phi c + e, g = Phi^T e, d = c -
 // w: p = w / S out, and the sums c.p, p.d, g.d by slices as above.  One pass and a
 // reduction in place of a launch per quotient, difference, product and sum (15 of
-// 36 launches of an evaluation: 60 rows, k = 20, R = 7, 215 -> 150 us from the host,
-// 94 -> 71 us in a graph).
+// 36 launches of an evaluation: 60 rows, k = 20, R = 7, 215 -> 141 us from the host,
+// 94 -> 74 us in a graph).
 __global__ __launch_bounds__(FT) void coef_part_kernel(size_t n, int R, int parts,
                                                        const double* __restrict__ c,
                                                        const double* __restrict__ g,

@@ -23,9 +23,9 @@ namespace rvgp {
 // the lanes look up a pop's edges together (hash table in LDS), and only those
 // that insert or decrease go to lane 0, in their order.  26 bytes a node and
 // 2 table entries: 32 wavefronts a CU at P = 128, 21 at 256, 10 at 512.
-// K = 15, k = 10 on a surface: 1993 -> 278 us at n = 5000, 5.5 -> 2.5 ms at
-// 100000; K = 30, k = 20 on a 3-torus, n = 100000: 20.9 -> 9.0 ms; K = 100 at
-// n = 5000 (P = 512): 23.7 -> 1.9 ms.
+// K = 15, k = 10 on a surface: 1950 -> 176 us at n = 5000, 5.5 -> 2.5 ms at
+// 100000; K = 30, k = 20 on a 3-torus, n = 100000: 20.9 -> 8.9 ms; K = 100 at
+// n = 5000 (P = 512): 23.7 -> 1.5 ms.
 template <int P>
 __global__ __launch_bounds__(64) void geo_nbh_wave_kernel(const int* __restrict__ rowptr,
                                                           const int* __restrict__ cols,
